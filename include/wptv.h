@@ -93,6 +93,7 @@ const char* wptv_last_error(void);
  *   splits     in: the number of parts each batch row's key range is cut
  *              into (0 = chosen from B, T, N and the GPU); the workspace must
  *              hold wptv_attention_workspace() bytes for the same arguments
+ *              (FP32 calls with a smaller one, or none, run in one part)
  *   out        [B, T, H, c] contiguous, dtype
  *   lse        NULL, or [B, T, H] fp32: each query head's natural-log
  *              log-sum-exp, the sink included

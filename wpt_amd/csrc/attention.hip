@@ -29,9 +29,11 @@
 //
 // Generic kernel (fp32 or bf16, any head width <= 256, chosen rows): one
 // wavefront per (batch row, query position, head), one key row per lane,
-// the reference algorithm in FP32 with an online softmax.  It is the fp32
-// path and the chosen-row (sparse) path.
-#include "wptv_common.h"
+// the reference algorithm in FP32 with an online softmax.  It serves what the
+// matrix-core kernels do not: chosen rows in FP32, other head widths, rows
+// that are not 16-byte aligned, scales of no bf16 kernel.  FP32 at head widths
+// 64 and 128 runs on attention_f32.hip.
+#include "attention_f32.h"
 
 #include <climits>
 #include <mutex>
@@ -39,106 +41,6 @@
 
 namespace wptv {
 namespace {
-
-constexpr float kNegInf = -__builtin_inff();
-
-struct Bounds {
-  int lo, hi;  // inclusive key-row range a query sees (hi < lo: none)
-};
-
-// The key rows query position t of batch row b sees, before the tree mask.
-// A batch row's query positions: p[t], or (a draft tree given without
-// positions) node t at base + t.
-// p[i] of an input that no kernel of the launch writes, read as constant
-// memory: a scalar load where i is uniform (on the scalar counter, apart from
-// the vector-memory counter the kernels' DMA runs on, which the compiler's own
-// waits cannot count), a vector load where it is not.
-template <typename T>
-__device__ __forceinline__ T const_load(const T* p, int64_t i) {
-  return ((const __attribute__((address_space(4))) T*)(uintptr_t)p)[i];
-}
-
-struct QueryPos {
-  const int64_t* p;
-  int64_t base;
-  __device__ __forceinline__ int64_t at(int t) const { return p ? const_load(p, t) : base + t; }
-};
-
-__device__ __forceinline__ QueryPos query_pos(const int64_t* positions, const int64_t* tree_base, int b, int T) {
-  return positions ? QueryPos{positions + (int64_t)b * T, 0} : QueryPos{nullptr, tree_base[b]};
-}
-
-__device__ __forceinline__ Bounds query_bounds(const QueryPos& pos_b, int t, int window, int N) {
-  const int64_t p = pos_b.at(t);
-  int64_t hi = p < (int64_t)N - 1 ? p : (int64_t)N - 1;
-  int64_t lo = window > 0 ? p - window + 1 : 0;
-  if (lo < 0) lo = 0;
-  Bounds r;
-  r.lo = (int)lo;
-  r.hi = hi < lo ? (int)lo - 1 : (int)hi;
-  return r;
-}
-
-// The union [u_lo, u_hi] of the key rows that positions t_first .. t_last
-// see (u_hi < u_lo: none), uniform.  A lane per position, so the positions
-// come in by one vector load instead of one dependent scalar load each; every
-// lane of the wavefront must be active.
-__device__ __forceinline__ void union_bounds(const QueryPos& pos_b, int t_first, int t_last, int window, int N,
-                                             int lane, int& u_lo, int& u_hi) {
-  int lo_l = INT_MAX, hi_l = -1;
-  for (int t0 = t_first; t0 <= t_last; t0 += 64) {
-    if (t0 + lane <= t_last) {
-      const Bounds bt = query_bounds(pos_b, t0 + lane, window, N);
-      if (bt.hi >= bt.lo) {
-        lo_l = min(lo_l, bt.lo);
-        hi_l = max(hi_l, bt.hi);
-      }
-    }
-  }
-  u_lo = __builtin_amdgcn_readfirstlane(wave_min_i32(lo_l));
-  u_hi = __builtin_amdgcn_readfirstlane(wave_max_i32(hi_l));
-}
-
-__device__ __forceinline__ bool tree_visible(int n, int64_t tbase, uint64_t anc) {
-  if ((int64_t)n < tbase) return true;
-  const int64_t node = (int64_t)n - tbase;
-  return node < 64 && ((anc >> node) & 1ull);
-}
-
-// Where logical row n (a token's position) of batch row b sits in the table:
-// physical row (n - base[b]) & mask.  The default (base NULL, mask all ones)
-// is token p at row p; a window layer's ring of 2^r rows per batch row has
-// mask 2^r - 1; a table that starts at a later token has base[b] = that
-// token's position.
-struct RowMap {
-  const int64_t* base;
-  uint32_t mask;
-};
-
-// The table row of batch row b's first ring slot (a scalar load).
-__device__ __forceinline__ int row_base(const RowMap& m, int b) { return m.base ? (int)const_load(m.base, b) : 0; }
-
-// A window or sparse layer's output gate (attention.py:128-130): the output
-// o (rounded to bf16, the attention's dtype) times sigmoid(gate) (rounded to
-// bf16, as torch.sigmoid of a bf16 tensor), rounded again.  Row (b*T + t) of
-// the gate at g + (b*T + t)*stride, head h's columns at + h*c; g NULL: none.
-struct OutGate {
-  const void* g;  // in the attention's dtype
-  int64_t stride;
-  template <typename E>
-  __device__ __forceinline__ const E* row(int b, int T, int r, int H, int C) const {
-    return g ? static_cast<const E*>(g) + ((int64_t)b * T + r / H) * stride + (int64_t)(r % H) * C : nullptr;
-  }
-};
-
-__device__ __forceinline__ float gate_factor(unsigned short g) {
-  return bf16_to_f32(f32_to_bf16(1.f / (1.f + __expf(-bf16_to_f32(g)))));
-}
-
-// o rounded to bf16, times the gate factor, rounded again.
-__device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) {
-  return f32_to_bf16(bf16_to_f32(f32_to_bf16(o)) * gate_factor(g));
-}
 
 // Merges the parts of one query row's 8 columns c8 .. c8 + 7: fixed split
 // order, log-sum-exp weights, the sink (log2 units; -inf: none) joining the
@@ -1901,7 +1803,7 @@ __global__ __launch_bounds__(64) void attention_generic(
 // Host side
 // ---------------------------------------------------------------------------
 
-enum Kind { kGeneric = 0, kRowBlocks = 1, kKeySplit = 2, kRowBlocks32 = 3 };
+enum Kind { kGeneric = 0, kRowBlocks = 1, kKeySplit = 2, kRowBlocks32 = 3, kF32Mfma = 4 };
 
 struct Plan {
   Kind kind;
@@ -1934,6 +1836,16 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
   if (c > kMaxC) return fail(WPTV_E_UNSUPPORTED, "verify_attention: head width %d above %d", c, kMaxC);
   Plan p{};
   const bool mfma = dtype == WPTV_BF16 && (c == 64 || c == 128) && !(flags & WPTV_ATTN_FORCE_GENERIC);
+  if (dtype == WPTV_F32 && attention_f32_takes(c) && !(flags & WPTV_ATTN_FORCE_GENERIC)) {
+    const F32Plan f = attention_f32_plan(B, T, H, c, N, window, requested);
+    p.kind = kF32Mfma;
+    p.mbw = 1;
+    p.groups = f.groups;
+    p.splits = f.splits;
+    p.bytes = f.bytes;
+    *out = p;
+    return WPTV_OK;
+  }
   if (!mfma) {
     p.kind = kGeneric;
     p.mbw = 0;
@@ -2067,8 +1979,18 @@ int attend(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
   int st = plan(B, T, H, c, N, window, dtype, flags, splits, &p);
   if (st != WPTV_OK) return st;
   const float scale_log2 = scale * kLog2e;
-  if (p.kind != kGeneric && !(scale > 0.f && scale < 1e30f)) p.kind = kGeneric, p.splits = 1, p.bytes = 0;  // the MFMA kernels take row maxima on unscaled scores
-  if (p.kind != kGeneric) {
+  if (p.kind == kF32Mfma) {
+    // 16-byte loads and stores of rows; without room for the parts, one part
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16) || k_stride_b % 4 ||
+        k_stride_n % 4 || v_stride_b % 4 || v_stride_n % 4)
+      p.kind = kGeneric, p.splits = 1, p.bytes = 0;
+    else if (p.bytes > 0 && (!workspace || workspace_bytes < p.bytes || !aligned(workspace, 16))) {
+      st = plan(B, T, H, c, N, window, dtype, flags, 1, &p);
+      if (st != WPTV_OK) return st;
+    }
+  } else if (p.kind != kGeneric && !(scale > 0.f && scale < 1e30f))
+    p.kind = kGeneric, p.splits = 1, p.bytes = 0;  // the MFMA kernels take row maxima on unscaled scores
+  if (p.kind != kGeneric && p.kind != kF32Mfma) {
     // 32-bit byte offsets within one batch row's table (buffer loads).
     const bool ok_range =
         (double)phys_rows * (double)(k_stride_n > v_stride_n ? k_stride_n : v_stride_n) * 2.0 < 4.0e9;
@@ -2081,6 +2003,20 @@ int attend(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
   if (out_fm && p.kind != kRowBlocks && p.kind != kRowBlocks32)
     return fail(WPTV_E_UNSUPPORTED, "verify_attention: the fm output layout needs the bf16 MFMA row-block kernel "
                                     "(head width 64 or 128, aligned operands, no key split)");
+  if (p.kind == kF32Mfma) {
+    const F32Plan f{p.groups, p.splits, p.bytes};
+    F32Call call{};
+    call.q = static_cast<const float*>(q), call.k = static_cast<const float*>(k);
+    call.v = static_cast<const float*>(v);
+    call.ksb = k_stride_b, call.ksn = k_stride_n, call.vsb = v_stride_b, call.vsn = v_stride_n;
+    call.positions = positions, call.tree_base = tree_base, call.ancestors = tree_ancestors, call.sink = sink;
+    call.row_base = rows.base, call.row_mask = rows.mask;
+    call.gate = static_cast<const float*>(gate.g), call.gate_stride = gate.stride;
+    call.B = B, call.T = T, call.H = H, call.c = c, call.N = N, call.window = window;
+    call.scale_log2 = scale_log2;
+    call.out = static_cast<float*>(out), call.lse = lse, call.workspace = workspace;
+    return attention_f32(f, call, stream);
+  }
   if (p.kind == kGeneric) {
     dim3 grid(T * H, B);
     if (dtype == WPTV_F32)
@@ -2269,6 +2205,8 @@ extern "C" int wptv_verify_attention_static(const void* q, const void* k, int64_
                                             hipStream_t stream) {
   Plan p;
   int st = plan(B, T, H, c, N, window, dtype, flags, splits, &p);
+  if (st == WPTV_OK && p.kind == kF32Mfma)  // FP32 calls keep no parts there, so that overlapping ones do not race
+    st = plan(B, T, H, c, N, window, dtype, flags, splits = 1, &p);
   if (st != WPTV_OK) return st;
   // a split count of the library's choosing steps down until its parts fit
   // the static array (one split needs none)

@@ -1,0 +1,113 @@
+// What the attention kernels share: the rows a query sees, where a logical row
+// sits in the table, and the output gate.
+#pragma once
+
+#include "wptv_common.h"
+
+#include <climits>
+
+namespace wptv {
+namespace {
+
+constexpr float kNegInf = -__builtin_inff();
+
+struct Bounds {
+  int lo, hi;  // inclusive key-row range a query sees (hi < lo: none)
+};
+
+// The key rows query position t of batch row b sees, before the tree mask.
+// A batch row's query positions: p[t], or (a draft tree given without
+// positions) node t at base + t.
+// p[i] of an input that no kernel of the launch writes, read as constant
+// memory: a scalar load where i is uniform (on the scalar counter, apart from
+// the vector-memory counter the kernels' DMA runs on, which the compiler's own
+// waits cannot count), a vector load where it is not.
+template <typename T>
+__device__ __forceinline__ T const_load(const T* p, int64_t i) {
+  return ((const __attribute__((address_space(4))) T*)(uintptr_t)p)[i];
+}
+
+struct QueryPos {
+  const int64_t* p;
+  int64_t base;
+  __device__ __forceinline__ int64_t at(int t) const { return p ? const_load(p, t) : base + t; }
+};
+
+__device__ __forceinline__ QueryPos query_pos(const int64_t* positions, const int64_t* tree_base, int b, int T) {
+  return positions ? QueryPos{positions + (int64_t)b * T, 0} : QueryPos{nullptr, tree_base[b]};
+}
+
+__device__ __forceinline__ Bounds query_bounds(const QueryPos& pos_b, int t, int window, int N) {
+  const int64_t p = pos_b.at(t);
+  int64_t hi = p < (int64_t)N - 1 ? p : (int64_t)N - 1;
+  int64_t lo = window > 0 ? p - window + 1 : 0;
+  if (lo < 0) lo = 0;
+  Bounds r;
+  r.lo = (int)lo;
+  r.hi = hi < lo ? (int)lo - 1 : (int)hi;
+  return r;
+}
+
+// The union [u_lo, u_hi] of the key rows that positions t_first .. t_last
+// see (u_hi < u_lo: none), uniform.  A lane per position, so the positions
+// come in by one vector load instead of one dependent scalar load each; every
+// lane of the wavefront must be active.
+__device__ __forceinline__ void union_bounds(const QueryPos& pos_b, int t_first, int t_last, int window, int N,
+                                             int lane, int& u_lo, int& u_hi) {
+  int lo_l = INT_MAX, hi_l = -1;
+  for (int t0 = t_first; t0 <= t_last; t0 += 64) {
+    if (t0 + lane <= t_last) {
+      const Bounds bt = query_bounds(pos_b, t0 + lane, window, N);
+      if (bt.hi >= bt.lo) {
+        lo_l = min(lo_l, bt.lo);
+        hi_l = max(hi_l, bt.hi);
+      }
+    }
+  }
+  u_lo = __builtin_amdgcn_readfirstlane(wave_min_i32(lo_l));
+  u_hi = __builtin_amdgcn_readfirstlane(wave_max_i32(hi_l));
+}
+
+__device__ __forceinline__ bool tree_visible(int n, int64_t tbase, uint64_t anc) {
+  if ((int64_t)n < tbase) return true;
+  const int64_t node = (int64_t)n - tbase;
+  return node < 64 && ((anc >> node) & 1ull);
+}
+
+// Where logical row n (a token's position) of batch row b sits in the table:
+// physical row (n - base[b]) & mask.  The default (base NULL, mask all ones)
+// is token p at row p; a window layer's ring of 2^r rows per batch row has
+// mask 2^r - 1; a table that starts at a later token has base[b] = that
+// token's position.
+struct RowMap {
+  const int64_t* base;
+  uint32_t mask;
+};
+
+// The table row of batch row b's first ring slot (a scalar load).
+__device__ __forceinline__ int row_base(const RowMap& m, int b) { return m.base ? (int)const_load(m.base, b) : 0; }
+
+// A window or sparse layer's output gate (attention.py:128-130): the output
+// o (rounded to bf16, the attention's dtype) times sigmoid(gate) (rounded to
+// bf16, as torch.sigmoid of a bf16 tensor), rounded again.  Row (b*T + t) of
+// the gate at g + (b*T + t)*stride, head h's columns at + h*c; g NULL: none.
+struct OutGate {
+  const void* g;  // in the attention's dtype
+  int64_t stride;
+  template <typename E>
+  __device__ __forceinline__ const E* row(int b, int T, int r, int H, int C) const {
+    return g ? static_cast<const E*>(g) + ((int64_t)b * T + r / H) * stride + (int64_t)(r % H) * C : nullptr;
+  }
+};
+
+__device__ __forceinline__ float gate_factor(unsigned short g) {
+  return bf16_to_f32(f32_to_bf16(1.f / (1.f + __expf(-bf16_to_f32(g)))));
+}
+
+// o rounded to bf16, times the gate factor, rounded again.
+__device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) {
+  return f32_to_bf16(bf16_to_f32(f32_to_bf16(o)) * gate_factor(g));
+}
+
+}  // namespace
+}  // namespace wptv
