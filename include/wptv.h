@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define WPTV_ABI_VERSION 10
+#define WPTV_ABI_VERSION 11
 
 enum {
   WPTV_OK = 0,
@@ -362,6 +362,11 @@ int wptv_gemm_parts(const void* x, int64_t ldx, const void* w, int64_t ldw, int 
  * rows 64 t + 32 .. 64 t + 63 their up rows (N a multiple of 64). */
 int wptv_gemm_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, int N, int K, void* out,
                      int64_t ldo, hipStream_t stream);
+
+/* wptv_gemm_wide_swiglu: the same on the 256 x 256 tiles, for any number of
+ * rows (a prompt's reading): N a multiple of 256, K of 32, ldo of 8. */
+int wptv_gemm_wide_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, int N, int K, void* out,
+                          int64_t ldo, hipStream_t stream);
 
 /* ---------------------------------------------------------------------------
  * The same products with fragment-major ("fm") operands, for the verify

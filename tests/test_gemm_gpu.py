@@ -149,3 +149,40 @@ def test_the_fused_swiglu_product_equals_the_product_then_swiglu(device, M):
     got = layers.linear_swiglu(x, layers.interleave_gate_up(w))
     assert got.shape == (M, F) and got.dtype == torch.bfloat16
     assert torch.equal(got, expected)
+
+
+@pytest.mark.parametrize("M,F,K", [(1, 128, 32), (257, 384, 96), (513, 128, 256), (2049, 512, 64), (2600, 384, 128)])
+def test_the_wide_swiglu_product_equals_the_wide_product_then_swiglu(device, M, F, K):
+    # tiles cut by the rows, chunk counts below the ring's depth, more row
+    # tiles than a band holds, tile counts the XCDs do not share evenly: bit
+    # for bit the wide product followed by wptv_swiglu
+    generator = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=generator).to(torch.bfloat16).to(device)
+    w = (torch.randn(2 * F, K, generator=generator) * 0.1).to(torch.bfloat16).to(device)
+    if M >= layers.WIDE_MIN_ROWS:
+        product = layers.linear(x, w)
+        # FP32 sums of K products of |x w| < 2, rounded to bf16 once: half a bf16 step of the largest result
+        assert relative_error(product.float().cpu(), (x.double() @ w.double().T).cpu()) < 2.0 ** -8
+    else:
+        product = (x.float() @ w.float().T).to(torch.bfloat16)
+    expected = layers.swiglu(product)
+    got = layers.linear_swiglu_wide(x, layers.interleave_gate_up(w))
+    assert got.shape == (M, F)
+    if M >= layers.WIDE_MIN_ROWS:
+        assert torch.equal(got, expected)
+    else:  # torch's FP32 product sums in another order: two bf16 steps
+        assert relative_error(got.float().cpu(), expected.float().cpu()) < 2.0 ** -7
+
+
+def test_the_wide_swiglu_product_writes_nothing_else(device):
+    from wpt_amd import _lib
+
+    M, F, K = 300, 128, 64
+    x, w = operands(M, 2 * F, K, seed=12, device=device)
+    wide = torch.full((M + 20, F + 8), 7.0, dtype=torch.bfloat16, device=device)
+    _lib.check(_lib.lib().wptv_gemm_wide_swiglu(x.data_ptr(), K, w.data_ptr(), K, M, 2 * F, K, wide.data_ptr(), F + 8,
+                                                _lib.stream(device)), "gemm_wide_swiglu")
+    assert torch.equal(wide[:M, :F], layers.linear_swiglu_wide(x, w))
+    assert (wide[M:] == 7).all() and (wide[:, F:] == 7).all()
+    with pytest.raises(NotImplementedError):
+        layers.linear_swiglu_wide(x, w[:192])  # 2F not a multiple of 256

@@ -12,7 +12,7 @@ from pathlib import Path
 import torch
 
 LIBRARY = Path(__file__).resolve().parent / "lib" / "libwptv.so"
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 WPTV_F32, WPTV_BF16 = 0, 1
 DTYPES = {torch.float32: WPTV_F32, torch.bfloat16: WPTV_BF16}
@@ -63,6 +63,7 @@ SIGNATURES = {
     "wptv_gemm_workspace": [_I, _I, _I, _P, _P],
     "wptv_gemm": [_P, _I64, _P, _I64, _I, _I, _I, _P, _I64, _I, _I, _P, _SZ, _P],
     "wptv_gemm_swiglu": [_P, _I64, _P, _I64, _I, _I, _I, _P, _I64, _P],
+    "wptv_gemm_wide_swiglu": [_P, _I64, _P, _I64, _I, _I, _I, _P, _I64, _P],
     "wptv_gemm_parts": [_P, _I64, _P, _I64, _I, _I, _I, _I, _P, _SZ, _P],
     "wptv_fm_pack": [_P, _I64, _I, _I, _I, _P, _P],
     "wptv_fm_row_blocks": [_I],

@@ -74,13 +74,6 @@ __device__ __forceinline__ void wait_chunks_behind(int behind) {
 
 enum GemmOut { kPartF32 = 0, kOutBf16 = 1, kOutF32 = 2, kOutSwiGLU = 3 };
 
-// silu(g) * u of the bf16-rounded halves, rounded once to bf16: what the
-// product rounded to bf16 and then wptv_swiglu give.
-__device__ __forceinline__ unsigned short swiglu_bf16(float g, float u) {
-  const float gb = bf16_to_f32(f32_to_bf16(g)), ub = bf16_to_f32(f32_to_bf16(u));
-  return f32_to_bf16(gb / (1.f + expf(-gb)) * ub);
-}
-
 // grid: (N / 64, splits).  Split z multiplies K chunks [z cps, min((z + 1) cps, K / 64)).
 // OUT: kPartF32 -> part[z][m][n] FP32; kOutBf16 -> out bf16; kOutF32 -> out
 // FP32 holding the bf16-rounded product (the reference's bf16 product cast to

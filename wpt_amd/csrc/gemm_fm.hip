@@ -60,11 +60,6 @@ __global__ __launch_bounds__(256) void fm_pack(const unsigned short* __restrict_
   *reinterpret_cast<u16x8*>(out + fm_offset(r, k, rb_count)) = v;
 }
 
-__device__ __forceinline__ unsigned short fm_swiglu_bf16(float g, float u) {
-  const float gb = bf16_to_f32(f32_to_bf16(g)), ub = bf16_to_f32(f32_to_bf16(u));
-  return f32_to_bf16(gb / (1.f + expf(-gb)) * ub);
-}
-
 // grid (N / (16 NB), splits, RBT / MB); split z takes k-steps [4 STEPS z, 4
 // STEPS (z + 1)), row group rg the row blocks [MB rg, MB (rg + 1)).  x: RBT
 // row blocks; w: NBT = N / 16 row blocks.  OUT kFmParts: part[z][m][n] FP32;
@@ -154,7 +149,7 @@ __global__ __launch_bounds__(kFmWaves * 64, 1) void gemm_fm(const u32x4* __restr
       const int pg = rb * NB + nb, pu = pg + 2;
       u16x4 res;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) res[i] = fm_swiglu_bf16(summed(pg, i), summed(pu, i));
+      for (int i = 0; i < 4; ++i) res[i] = swiglu_bf16(summed(pg, i), summed(pu, i));
       *reinterpret_cast<u16x4*>(static_cast<unsigned short*>(out) + fm_offset(m, tile * 8 * NB + gb * 16 + 4 * g, RBT)) =
           res;
     }

@@ -35,9 +35,26 @@
 // lane along whole output rows, as bf16 or as the bf16 values widened to FP32
 // (the reference's .float() of the bf16 logits).
 //
-// Workgroups are dealt to the 8 XCDs in turn; the row tiles of one column tile
-// take consecutive slots of one XCD, so its weights come from HBM once and
-// from that XCD's L2 for the other row tiles.
+// The feed-forward block's gate/up product of a prompt's reading stores
+// silu(gate) * up instead of the product (kWideSwiGLU).  Measured on the MI355X
+// at 4096 rows, 11264 x 2048, us: 197 (half of the product's bytes leave, the
+// SwiGLU runs on what the registers hold) against 311 for hipBLASLt's product
+// (155) and torch's four passes over its halves; 62 against 95 at 1000 rows, 52
+// against 64 at 513.
+//
+// Where the time goes, 4096 rows x 32768 x 2048 and 8192^3 (us): as it is 535,
+// 872; without the DMA 405, 640 (the rate the matrix cores hold on random data);
+// without the products 464, 750; so the operands' 32 KiB a chunk, not the
+// products, set the pace (fm operands, contiguous KiB, 480, 805).  Not kept:
+// one workgroup a compute unit walking the tiles with the next tile's chunks
+// requested ahead and results stored from a staging of their own (538, 895: the
+// tiles' ends are not what costs); four wavefronts of 128 x 128 with the LDS
+// reads between the products (563, 930); a fifth ring slot (the same); the DMA
+// issued among the products (553, 920).
+//
+// Tiles in bands of 8 rows, an XCD's in one run (wide_tile_of): 8192^3 1378 ->
+// 865 us, 4096 x 32768 x 2048 550 -> 523 us against a column's row tiles on one
+// XCD; at 496 rows (two row tiles) the two are alike.
 #include "wptv_common.h"
 
 #include <climits>
@@ -87,7 +104,11 @@ __device__ __forceinline__ void wait_lgkm0() {
 // the tile's 256 columns and its first index, as a (value, index) pair at
 // out[column tile * M + row] (the greedy decisions' first maximal index,
 // reduced over the column tiles by wide_argmax_reduce).
-enum WideOut { kWideBf16 = 0, kWideF32 = 1, kWideArgmax = 2 };
+// kWideSwiGLU: w's rows are gate and up rows interleaved by 32
+// (wptv_gemm_swiglu's order), so a wavefront's two 32-column blocks are 32
+// features' gates and ups, register for register; out holds silu(gate) * up
+// (both rounded to bf16 first, as the product's are), [M, N / 2] bf16.
+enum WideOut { kWideBf16 = 0, kWideF32 = 1, kWideArgmax = 2, kWideSwiGLU = 3 };
 
 // torch.argmax's order: a NaN above every number, then the larger value;
 // the lower index among equals (NaNs included).
@@ -99,6 +120,21 @@ __device__ __forceinline__ void wide_better(float& v, int& i, float v2, int i2) 
   }
 }
 
+// Workgroup id's tile.  Workgroups are dealt to the 8 XCDs in turn; each XCD
+// takes one run of consecutive tiles, in bands of up to 8 row tiles walked
+// column by column, so the 32 tiles an XCD works on at a time are about 8 x 4:
+// each of its L2's lines of X and W serves 4 and 8 of them.
+__device__ __forceinline__ void wide_tile_of(int id, int row_tiles, int col_tiles, int& rt, int& ct) {
+  constexpr int kBand = 8;
+  const int total = row_tiles * col_tiles, q = total / 8, r = total % 8;
+  const int xcd = id & 7;
+  const int tile = xcd * q + min(xcd, r) + (id >> 3);
+  const int band = tile / (kBand * col_tiles), in_band = tile - band * kBand * col_tiles;
+  const int rows = min(kBand, row_tiles - band * kBand);
+  rt = band * kBand + in_band % rows;
+  ct = in_band / rows;
+}
+
 template <int OUT, bool FM>
 __global__ __launch_bounds__(kWideWaves * 64, 1) void gemm_wide(const unsigned short* __restrict__ x, int64_t ldx,
                                                                 const unsigned short* __restrict__ w, int64_t ldw,
@@ -108,19 +144,8 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void gemm_wide(const unsigned s
 
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col_tiles = N / kWideTile;
   int rt, ct;
-  {
-    const int id = blockIdx.x;
-    if (col_tiles % 8 == 0) {  // slot s of XCD x: column tile 8 (s / row_tiles) + x, row tile s % row_tiles
-      const int xcd = id & 7, slot = id >> 3;
-      rt = slot % row_tiles;
-      ct = (slot / row_tiles) * 8 + xcd;
-    } else {
-      rt = id % row_tiles;
-      ct = id / row_tiles;
-    }
-  }
+  wide_tile_of(blockIdx.x, row_tiles, N / kWideTile, rt, ct);
   const int m0 = rt * kWideTile, n0 = ct * kWideTile;
   const int chunks = K / kWideChunk;
 
@@ -195,7 +220,6 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void gemm_wide(const unsigned s
   // the barrier before phase 2 s; its slot is refilled (chunk s + 4) from
   // phase 2 s + 2 on, after both groups have read it.
   auto load = [&](int c) {
-    issue(c + 3);
     const unsigned char* st = ring + (c % kWideStages) * kWideStage;
 #pragma unroll
     for (int kk = 0; kk < kWideSlices; ++kk) {
@@ -206,6 +230,8 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void gemm_wide(const unsigned s
       for (int i = 0; i < 4; ++i)
         xf[kk][i] = *reinterpret_cast<const bf16x8*>(st + xbase + (uint32_t)(32 * i) * kWideRow + koff[kk]);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    issue(c + 3);  // while the fragments come in
     wait_lgkm0();  // the slot may be refilled once both groups have passed the next barriers
   };
   auto multiply = [&]() {
@@ -297,31 +323,43 @@ __global__ __launch_bounds__(kWideWaves * 64, 1) void gemm_wide(const unsigned s
   // every wavefront is done with the ring: stage the tile as bf16 [m][n]
   __syncthreads();
   typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+  constexpr int kPieces = OUT == kWideSwiGLU ? 16 : 32;  // 16-byte pieces of a staged row
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int i = 0; i < 4; ++i) {
+    const int ml = 128 * wm + 32 * i + rl;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ml = 128 * wm + 32 * i + rl;
+    for (int g = 0; g < 4; ++g) {
+      if constexpr (OUT == kWideSwiGLU) {
+        const int q = 4 * wn + g;  // features 32 wn + 8 g .. + 7 of the tile
+        u16x4 v;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int q = 8 * wn + 4 * j + g;  // 16-byte piece of row ml: columns 8 q .. 8 q + 7
-        const u16x4 v = {f32_to_bf16(acc[j][i][4 * g]), f32_to_bf16(acc[j][i][4 * g + 1]),
-                         f32_to_bf16(acc[j][i][4 * g + 2]), f32_to_bf16(acc[j][i][4 * g + 3])};
-        *reinterpret_cast<u16x4*>(ring + ml * 512 + 16 * (q ^ (ml & 7)) + 8 * hl) = v;
+        for (int e = 0; e < 4; ++e) v[e] = swiglu_bf16(acc[0][i][4 * g + e], acc[1][i][4 * g + e]);
+        *reinterpret_cast<u16x4*>(ring + ml * (16 * kPieces) + 16 * (q ^ (ml & 7)) + 8 * hl) = v;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int q = 8 * wn + 4 * j + g;  // columns 8 q .. 8 q + 7 of the tile
+          const u16x4 v = {f32_to_bf16(acc[j][i][4 * g]), f32_to_bf16(acc[j][i][4 * g + 1]),
+                           f32_to_bf16(acc[j][i][4 * g + 2]), f32_to_bf16(acc[j][i][4 * g + 3])};
+          *reinterpret_cast<u16x4*>(ring + ml * (16 * kPieces) + 16 * (q ^ (ml & 7)) + 8 * hl) = v;
+        }
       }
     }
+  }
   __syncthreads();
-  const int q = threadIdx.x & 31;
+  constexpr int kRowsAtOnce = kWideWaves * 64 / kPieces;
+  const int q = threadIdx.x % kPieces;
+  const int64_t col0 = OUT == kWideSwiGLU ? n0 / 2 : n0;
 #pragma unroll 4
-  for (int pass = 0; pass < kWideTile / 16; ++pass) {
-    const int ml = 16 * pass + (threadIdx.x >> 5);
+  for (int pass = 0; pass < kWideTile / kRowsAtOnce; ++pass) {
+    const int ml = kRowsAtOnce * pass + threadIdx.x / kPieces;
     const int m = m0 + ml;
     if (m >= M) break;
-    const u16x8 v = *reinterpret_cast<const u16x8*>(ring + ml * 512 + 16 * (q ^ (ml & 7)));
-    if constexpr (OUT == kWideBf16) {
-      *reinterpret_cast<u16x8*>(static_cast<unsigned short*>(out) + (int64_t)m * ldo + n0 + 8 * q) = v;
+    const u16x8 v = *reinterpret_cast<const u16x8*>(ring + ml * (16 * kPieces) + 16 * (q ^ (ml & 7)));
+    if constexpr (OUT != kWideF32) {
+      *reinterpret_cast<u16x8*>(static_cast<unsigned short*>(out) + (int64_t)m * ldo + col0 + 8 * q) = v;
     } else {
-      float* dst = static_cast<float*>(out) + (int64_t)m * ldo + n0 + 8 * q;
+      float* dst = static_cast<float*>(out) + (int64_t)m * ldo + col0 + 8 * q;
       *reinterpret_cast<f32x4*>(dst) = f32x4{bf16_to_f32(v[0]), bf16_to_f32(v[1]), bf16_to_f32(v[2]), bf16_to_f32(v[3])};
       *reinterpret_cast<f32x4*>(dst + 4) =
           f32x4{bf16_to_f32(v[4]), bf16_to_f32(v[5]), bf16_to_f32(v[6]), bf16_to_f32(v[7])};
@@ -358,7 +396,9 @@ bool gemm_wide_fits(int M, int N, int K) { return M > 0 && N > 0 && K > 0 && N %
 // dimensions multiples of 8, operands under 4 GB.
 namespace {
 
-constexpr int kWideArgmaxOut = -100;  // launch_wide's out_dtype for the argmax epilogue
+// launch_wide's out_dtype for the epilogues that store something else
+constexpr int kWideArgmaxOut = -100;
+constexpr int kWideSwiGLUOut = -101;
 
 template <bool FM>
 int launch_wide(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, int N, int K, void* out, int64_t ldo,
@@ -368,7 +408,11 @@ int launch_wide(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, i
   if (groups > 0x7fffffffLL) return fail(WPTV_E_UNSUPPORTED, "gemm: %lld output tiles", groups);
   const auto* xb = static_cast<const unsigned short*>(x);
   const auto* wb = static_cast<const unsigned short*>(w);
-  if (out_dtype == kWideArgmaxOut)
+  if (out_dtype == kWideSwiGLUOut) {
+    if constexpr (!FM)
+      hipLaunchKernelGGL((gemm_wide<kWideSwiGLU, FM>), dim3((unsigned)groups), dim3(kWideWaves * 64), 0, stream, xb,
+                         ldx, wb, ldw, M, N, K, row_tiles, out, ldo);
+  } else if (out_dtype == kWideArgmaxOut)
     hipLaunchKernelGGL((gemm_wide<kWideArgmax, FM>), dim3((unsigned)groups), dim3(kWideWaves * 64), 0, stream, xb,
                        ldx, wb, ldw, M, N, K, row_tiles, out, ldo);
   else if (out_dtype == WPTV_BF16)
@@ -394,6 +438,21 @@ int gemm_wide(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, int
 }  // namespace wptv
 
 using namespace wptv;
+
+extern "C" int wptv_gemm_wide_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw, int M, int N, int K,
+                                     void* out, int64_t ldo, hipStream_t stream) {
+  if (!x || !w || !out) return fail(WPTV_E_INVALID, "gemm_wide_swiglu: x, w and out must be given");
+  if (!gemm_wide_fits(M, N, K))
+    return fail(WPTV_E_UNSUPPORTED, "gemm_wide_swiglu: M > 0, N a multiple of %d and K of %d (got %d, %d, %d)",
+                kWideTile, kWideChunk, M, N, K);
+  if (ldx < K || ldw < K || ldo < N / 2)
+    return fail(WPTV_E_INVALID, "gemm_wide_swiglu: a leading dimension below the row width");
+  if (!aligned(x, 16) || !aligned(w, 16) || !aligned(out, 16) || ldx % 8 || ldw % 8 || ldo % 8)
+    return fail(WPTV_E_INVALID, "gemm_wide_swiglu: x, w and out 16-byte aligned, leading dimensions of 8 elements");
+  if ((double)N * (double)ldw * 2.0 >= 4.0e9 || (double)M * (double)ldx * 2.0 >= 4.0e9)
+    return fail(WPTV_E_UNSUPPORTED, "gemm_wide_swiglu: operands above 4 GB");
+  return launch_wide<false>(x, ldx, w, ldw, M, N, K, out, ldo, kWideSwiGLUOut, stream);
+}
 
 extern "C" int wptv_gemm_fm_wide(const void* x_fm, int x_blocks, const void* w_fm, int M, int N, int K, void* out,
                                  int64_t ldo, int out_dtype, hipStream_t stream) {

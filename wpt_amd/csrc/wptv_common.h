@@ -91,6 +91,13 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
+// silu(g) * u of the bf16-rounded halves, rounded once to bf16: what the
+// product rounded to bf16 and then wptv_swiglu give.
+__device__ __forceinline__ unsigned short swiglu_bf16(float g, float u) {
+  const float gb = bf16_to_f32(f32_to_bf16(g)), ub = bf16_to_f32(f32_to_bf16(u));
+  return f32_to_bf16(gb / (1.f + expf(-gb)) * ub);
+}
+
 __device__ __forceinline__ float wave_max(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));

@@ -37,7 +37,8 @@ On the GPU:
                     block; wptv_gemm's split-K parts otherwise up to
                     SPLIT_K_ROWS bf16 rows (summed by qkv_post and the
                     residual add + norm), the gate/up product with SwiGLU in
-                    its epilogue (wptv_gemm_swiglu) at up to 512 bf16 rows;
+                    its epilogue (wptv_gemm_swiglu at up to 512 bf16 rows,
+                    the 256 x 256 tiles of wptv_gemm_wide_swiglu above);
                     the lm_head on wptv_gemm (the skinny products up to 320
                     rows, the 256 x 256 tiles above); hipBLASLt only for a
                     prefill's wider layer products
@@ -260,7 +261,9 @@ class MQADecoder:
             act = layers.swiglu(F.linear(x, w[f"layers.{i}.gate_up"]))
         elif B * T <= layers.LINEAR_MAX_ROWS:
             act = layers.linear_swiglu(x, w[f"layers.{i}.gate_up_tiles"])  # SwiGLU in the product's epilogue
-        else:  # wider readings (a prefill): the product, then SwiGLU of its tile-interleaved halves
+        elif layers.wide_tiles(B * T, 2 * self.config.ffn, self.config.d_model):  # a prompt's reading
+            act = layers.linear_swiglu_wide(x, w[f"layers.{i}.gate_up_tiles"])
+        else:  # widths the tiles do not divide: the product, then SwiGLU of its tile-interleaved halves
             gu = F.linear(x, w[f"layers.{i}.gate_up_tiles"]).unflatten(-1, (-1, 2, 32))
             act = (F.silu(gu[..., 0, :].float()) * gu[..., 1, :].float()).flatten(-2).to(x.dtype)
         down = w[f"layers.{i}.down"]

@@ -249,6 +249,26 @@ def linear_swiglu(x, w_interleaved):
     return out.reshape(*x.shape[:-1], N // 2)
 
 
+def linear_swiglu_wide(x, w_interleaved):
+    """linear_swiglu on the 256 x 256 tiles (wptv_gemm_wide_swiglu), for any
+    number of rows: 2F a multiple of 256, K of 32."""
+    _gpu(x, w_interleaved)
+    if x.dtype != torch.bfloat16 or w_interleaved.dtype != torch.bfloat16:
+        raise ValueError(f"linear_swiglu_wide takes bf16 operands; got {x.dtype} and {w_interleaved.dtype}")
+    K = x.shape[-1]
+    N = w_interleaved.shape[0]
+    if w_interleaved.dim() != 2 or w_interleaved.shape[1] != K or w_interleaved.stride(1) != 1:
+        raise ValueError(f"w must be (2F, K={K}) with contiguous rows; got {tuple(w_interleaved.shape)}")
+    x2 = x.reshape(-1, K)
+    if x2.stride(1) != 1:
+        x2 = x2.contiguous()
+    M = x2.shape[0]
+    out = torch.empty(M, N // 2, dtype=torch.bfloat16, device=x.device)
+    check(_lib.lib().wptv_gemm_wide_swiglu(ptr(x2), x2.stride(0), ptr(w_interleaved), w_interleaved.stride(0), M, N,
+                                           K, ptr(out), out.stride(0), _lib.stream(x.device)), "gemm_wide_swiglu")
+    return out.reshape(*x.shape[:-1], N // 2)
+
+
 def linear_parts(x, w, splits=0, max_splits=8):
     """The split-K parts of x (..., K) . w (N, K)^T: FP32 (S, rows, N) whose
     sum over S is the product (wptv_gemm_parts), for a consumer that sums them
