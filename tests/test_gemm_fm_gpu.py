@@ -219,3 +219,24 @@ def test_the_fused_head_argmax_is_the_argmax_of_the_bf16_logits(device, M, N, K)
     assert torch.equal(best, expected)
     assert best[1] == 0 and torch.isnan(logits[2]).any()
     assert (best[rows_tied[(rows_tied != 1) & (rows_tied != 2)]] == 5).all()
+
+
+@pytest.mark.parametrize("M", [161, 192, 193, 224, 235, 256, 257, 288])
+def test_the_products_between_160_and_289_rows(device, M):
+    # each row-group form at its smallest and largest row count: the parts
+    # against an FP32 product, SwiGLU in place of the down product's operand
+    for N, K in ((2304, 2048), (2048, 5632), (64, 256)):
+        x, w = operands(M, N, K, seed=M + N, device=device)
+        parts = layers.linear_fm_parts(layers.fm_pack(x), M, layers.FmWeight(w), any_rows=True)
+        assert relative_error(parts.sum(0).cpu(), (x.float() @ w.float().T).cpu()) < 1e-5
+    F, K = 352, 2048
+    x, w = operands(M, 2 * F, K, seed=M, device=device)
+    out = layers.linear_fm_swiglu(layers.fm_pack(x), M, layers.FmWeight(layers.interleave_gate_up(w)), any_rows=True)
+    product = (x.float() @ w.float().T).to(torch.bfloat16).float()
+    g, u = product[:, :F], product[:, F:]
+    expected = (g * torch.sigmoid(g) * u).cpu()
+    # the gate and up sums may round to neighbouring bf16 values (2^-8 each), the result rounds once more
+    error = (layers.fm_unpack(out, M, F).float().cpu() - expected).abs()
+    assert (error <= 2.0 ** -6 * expected.abs() + 1e-6).all()
+    with pytest.raises(NotImplementedError):
+        layers.linear_fm_parts(layers.fm_pack(x), M, layers.FmWeight(w[:, :].contiguous()))

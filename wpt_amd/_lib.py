@@ -70,6 +70,9 @@ SIGNATURES = {
     "wptv_gemm_fm_plan": [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_SZ)],
     "wptv_gemm_fm_parts": [_P, _P, _I, _I, _I, _I, _P, _SZ, _P],
     "wptv_gemm_fm_swiglu": [_P, _P, _I, _I, _I, _P, _P],
+    "wptv_gemm_fm_any_plan": [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_SZ)],
+    "wptv_gemm_fm_any_parts": [_P, _P, _I, _I, _I, _I, _P, _SZ, _P],
+    "wptv_gemm_fm_any_swiglu": [_P, _P, _I, _I, _I, _P, _P],
     "wptv_gemm_fm_wide": [_P, _I, _P, _I, _I, _I, _P, _I64, _I, _P],
     "wptv_gemm_fm_wide_argmax_workspace": [_I, _I, _P],
     "wptv_gemm_fm_wide_argmax": [_P, _I, _P, _I, _I, _I, _P, _P, _SZ, _P],

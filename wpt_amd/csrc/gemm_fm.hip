@@ -3,7 +3,7 @@
 //   C[M, N] = X[M, K] . W[N, K]^T       bf16 in, FP32 accumulation
 //
 // the reference's projections under bf16 autocast (attention.py:157-168,
-// layers.py:45-61) at M = B (k+1) <= 160 rows.  Both operands are stored in
+// layers.py:45-61) at M = B (k+1) <= 320 rows.  Both operands are stored in
 // the fm layout (wptv_common.h: 1 KiB blocks of 16 rows x 32 columns in the
 // register order of v_mfma_f32_16x16x32_bf16): the weights packed once
 // (wptv_fm_pack), X written that way by the kernel that produces it (the
@@ -18,7 +18,8 @@
 // W through each compute unit for the same workgroup count: measured on the
 // MI355X with cold weights, q/k/v 6.4 against 7.2 us, output 5.7 against 5.9,
 // down 10.9 against 12.2, gate/up 18.9 against 20.0; at 320 rows each
-// quarter, 80 rows by 128 columns, and 80 by 64 for gate/up); its wavefronts
+// quarter, 80 rows by 128 columns, and 80 by 64 for gate/up; between, fm_plan);
+// its wavefronts
 // share out the part's 32-wide k-steps (wave w takes k-steps w, w + 4, ...),
 // each multiplying the group's rows by the NB column blocks:
 //
@@ -167,11 +168,13 @@ bool fm_steps_built(int s) {
 
 struct FmPlan {
   int mb, nb, splits, steps;
-  int groups;  // row groups of mb row blocks: 2 at 160 rows, 4 at 320, else 1
+  int groups;  // row groups of mb row blocks: 1 up to 128 rows, else 2 or 4
   size_t bytes;
 };
 
-int fm_plan(int M, int N, int K, bool swiglu, int requested, FmPlan* p) {
+// halves: 161 to 288 rows are taken too (in two row groups; gate/up at 256
+// rows in four).
+int fm_plan(int M, int N, int K, bool swiglu, bool halves, int requested, FmPlan* p) {
   if (M <= 0 || N <= 0 || K <= 0)
     return fail(WPTV_E_INVALID, "gemm_fm: M, N and K must be positive (got %d, %d, %d)", M, N, K);
   if (M > kFmMaxRows) return fail(WPTV_E_UNSUPPORTED, "gemm_fm: M = %d above %d rows", M, kFmMaxRows);
@@ -219,6 +222,17 @@ int fm_plan(int M, int N, int K, bool swiglu, int requested, FmPlan* p) {
     p->mb = 5;
     p->nb = swiglu ? nb : 4 * nb;
     p->groups = 4;
+  } else if (halves && rb > 10 && rb < 20 && N % 64 == 0) {
+    // 161 to 288 rows: halves by 64 columns, the most rows that share a
+    // workgroup's weights (the SwiGLU form at 256 rows: quarters, two workgroups
+    // a compute unit).  Measured on the MI355X with cold weights, q/k/v, output,
+    // gate/up, down in us, against the row-major products: 235 rows 7.8, 6.4,
+    // 27.5, 13.0 against 11.0, 11.2, 36.4, 15.1 (traced); of the other
+    // tilings (rows of 3, 4, 6 blocks by 32, 64 or 128 columns) none was more
+    // than 0.7 us faster at a product
+    p->mb = swiglu && rb == 16 ? 4 : rb / 2;
+    p->nb = 4;
+    p->groups = rb / p->mb;
   } else if (rb > 10) {
     return fail(WPTV_E_UNSUPPORTED, "gemm_fm: %d rows have no kernel form (up to 160, or 289 to 320)", M);
   }
@@ -252,6 +266,15 @@ template <int NB, int OUT>
 int launch_fm(const FmPlan& p, hipStream_t stream, const void* x, const void* w, int M, int N, void* out) {
   const int NBT = N / 16, RBT = fm_row_blocks(M);
   const dim3 grid(N / (16 * p.nb), p.splits, p.groups);
+  if (p.groups > 1 && p.mb != 5) {
+    switch (p.mb) {
+      case 4: return launch_fm_steps<4, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
+      case 6: return launch_fm_steps<6, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
+      case 7: return launch_fm_steps<7, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
+      case 8: return launch_fm_steps<8, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
+      default: return launch_fm_steps<9, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
+    }
+  }
   if (p.groups > 1) {  // groups of 5 row blocks by 4 or 8 column blocks
     if (p.nb == 4) return launch_fm_steps<5, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
     return launch_fm_steps<5, 8, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
@@ -292,21 +315,23 @@ extern "C" int wptv_fm_pack(const void* a, int64_t lda, int rows, int K, int row
 
 extern "C" int wptv_fm_row_blocks(int M) { return fm_row_blocks(M); }
 
-extern "C" int wptv_gemm_fm_plan(int M, int N, int K, int swiglu, int* splits, size_t* parts_bytes) {
+namespace {
+
+int fm_plan_out(int M, int N, int K, bool swiglu, bool halves, int* splits, size_t* parts_bytes) {
   if (!splits || !parts_bytes) return fail(WPTV_E_INVALID, "gemm_fm_plan: null output pointer");
   FmPlan p;
-  const int st = fm_plan(M, N, K, swiglu != 0, *splits, &p);
+  const int st = fm_plan(M, N, K, swiglu, halves, *splits, &p);
   if (st != WPTV_OK) return st;
   *splits = p.splits;
   *parts_bytes = p.bytes;
   return WPTV_OK;
 }
 
-extern "C" int wptv_gemm_fm_parts(const void* x_fm, const void* w_fm, int M, int N, int K, int splits, float* parts,
-                                  size_t parts_bytes, hipStream_t stream) {
+int fm_parts(const void* x_fm, const void* w_fm, int M, int N, int K, bool halves, int splits, float* parts,
+             size_t parts_bytes, hipStream_t stream) {
   if (!x_fm || !w_fm || !parts) return fail(WPTV_E_INVALID, "gemm_fm_parts: x, w and parts must be given");
   FmPlan p;
-  const int st = fm_plan(M, N, K, false, splits, &p);
+  const int st = fm_plan(M, N, K, false, halves, splits, &p);
   if (st != WPTV_OK) return st;
   if (splits <= 0) return fail(WPTV_E_INVALID, "gemm_fm_parts: take the part count from wptv_gemm_fm_plan");
   if (!fm_operands_ok(x_fm, w_fm, N, K) || !aligned(parts, 16))
@@ -316,13 +341,42 @@ extern "C" int wptv_gemm_fm_parts(const void* x_fm, const void* w_fm, int M, int
   return launch_fm<2, kFmParts>(p, stream, x_fm, w_fm, M, N, parts);
 }
 
-extern "C" int wptv_gemm_fm_swiglu(const void* x_fm, const void* w_fm, int M, int N, int K, void* out_fm,
-                                   hipStream_t stream) {
+int fm_swiglu(const void* x_fm, const void* w_fm, int M, int N, int K, bool halves, void* out_fm, hipStream_t stream) {
   if (!x_fm || !w_fm || !out_fm) return fail(WPTV_E_INVALID, "gemm_fm_swiglu: x, w and out must be given");
   FmPlan p;
-  const int st = fm_plan(M, N, K, true, 1, &p);
+  const int st = fm_plan(M, N, K, true, halves, 1, &p);
   if (st != WPTV_OK) return st;
   if (!fm_operands_ok(x_fm, w_fm, N, K) || !aligned(out_fm, 8))
     return fail(WPTV_E_INVALID, "gemm_fm_swiglu: x and w 16-byte aligned (out 8), w under 4 GB");
   return launch_fm<4, kFmSwiGLU>(p, stream, x_fm, w_fm, M, N, out_fm);
+}
+
+}  // namespace
+
+extern "C" int wptv_gemm_fm_plan(int M, int N, int K, int swiglu, int* splits, size_t* parts_bytes) {
+  return fm_plan_out(M, N, K, swiglu != 0, false, splits, parts_bytes);
+}
+
+extern "C" int wptv_gemm_fm_parts(const void* x_fm, const void* w_fm, int M, int N, int K, int splits, float* parts,
+                                  size_t parts_bytes, hipStream_t stream) {
+  return fm_parts(x_fm, w_fm, M, N, K, false, splits, parts, parts_bytes, stream);
+}
+
+extern "C" int wptv_gemm_fm_swiglu(const void* x_fm, const void* w_fm, int M, int N, int K, void* out_fm,
+                                   hipStream_t stream) {
+  return fm_swiglu(x_fm, w_fm, M, N, K, false, out_fm, stream);
+}
+
+extern "C" int wptv_gemm_fm_any_plan(int M, int N, int K, int swiglu, int* splits, size_t* parts_bytes) {
+  return fm_plan_out(M, N, K, swiglu != 0, true, splits, parts_bytes);
+}
+
+extern "C" int wptv_gemm_fm_any_parts(const void* x_fm, const void* w_fm, int M, int N, int K, int splits,
+                                      float* parts, size_t parts_bytes, hipStream_t stream) {
+  return fm_parts(x_fm, w_fm, M, N, K, true, splits, parts, parts_bytes, stream);
+}
+
+extern "C" int wptv_gemm_fm_any_swiglu(const void* x_fm, const void* w_fm, int M, int N, int K, void* out_fm,
+                                       hipStream_t stream) {
+  return fm_swiglu(x_fm, w_fm, M, N, K, true, out_fm, stream);
 }

@@ -29,7 +29,7 @@ On the GPU:
     the lengths     wptv_cache_lengths after the reading and after an undo
     verify attention wptv_verify_attention, reading only the rows the query
                     positions reach in the cache's table
-    projections     the matrix products of the dtype on MFMA: at up to 160
+    projections     the matrix products of the dtype on MFMA: at up to 320
                     bf16 rows the fragment-major products (wptv_gemm_fm_*:
                     weights packed once, X written in that layout by the
                     norms, the attention and the SwiGLU epilogue) for the
@@ -218,11 +218,12 @@ class MQADecoder:
 
     def fm_rows(self, rows):
         """Whether a reading of `rows` rows runs the fm products (bf16, up to
-        160 rows or 289 to 320, every layer's shapes taken by a kernel form)."""
+        320 rows, every layer's shapes taken by a kernel form)."""
         ok = self._fm_rows.get(rows)
         if ok is None:
             ok = self.dtype == torch.bfloat16 and all(
-                layers.fm_plan(rows, w.shape[0], w.shape[1], swiglu=name.endswith("gate_up_tiles")) is not None
+                layers.fm_plan(rows, w.shape[0], w.shape[1], swiglu=name.endswith("gate_up_tiles"),
+                               any_rows=True) is not None
                 for name, w in self.fm.items())
             self._fm_rows[rows] = ok
         return ok
@@ -252,10 +253,10 @@ class MQADecoder:
         else:
             handoff = self._exact_attention(i, h, x_in, cache, positions, counts, xf)
         if fm:
-            act = layers.linear_fm_swiglu(xf, B * T, self.fm[f"layers.{i}.gate_up_tiles"])
+            act = layers.linear_fm_swiglu(xf, B * T, self.fm[f"layers.{i}.gate_up_tiles"], any_rows=True)
             nxt = self._attn_input_fm(i + 1, fm)
-            layers.add_rms_norm_parts(h, layers.linear_fm_parts(act, B * T, self.fm[f"layers.{i}.down"]), next_norm,
-                                      xf if nxt else x, fm=nxt)
+            down = layers.linear_fm_parts(act, B * T, self.fm[f"layers.{i}.down"], any_rows=True)
+            layers.add_rms_norm_parts(h, down, next_norm, xf if nxt else x, fm=nxt)
             return handoff
         if x.dtype != torch.bfloat16:
             act = layers.swiglu(F.linear(x, w[f"layers.{i}.gate_up"]))
@@ -289,7 +290,7 @@ class MQADecoder:
             B, T, D = h.shape
             rows = B * T
             if o.dim() == 1:
-                parts = layers.linear_fm_parts(o, rows, self.fm[f"layers.{i}.out"])
+                parts = layers.linear_fm_parts(o, rows, self.fm[f"layers.{i}.out"], any_rows=True)
             else:
                 parts = layers.linear_parts(o.reshape(rows, -1), self.w[f"layers.{i}.out"])
             layers.add_rms_norm_parts(h, parts, self.w[f"layers.{i}.ffn_norm"], xf, fm=True)
@@ -345,7 +346,7 @@ class MQADecoder:
         # parts summed by the kernel that consumes them; torch's otherwise
         few = h.dtype == torch.bfloat16 and B * T <= SPLIT_K_ROWS
         if fm:
-            q = layers.qkv_post_parts(layers.linear_fm_parts(xf, B * T, self.fm[f"layers.{i}.qkv"]),
+            q = layers.qkv_post_parts(layers.linear_fm_parts(xf, B * T, self.fm[f"layers.{i}.qkv"], any_rows=True),
                                       w[f"layers.{i}.q_norm"], w[f"layers.{i}.k_norm"], table, cache.lengths, counts,
                                       H, T)
         elif few:

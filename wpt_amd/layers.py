@@ -318,7 +318,7 @@ def add_rms_norm_parts(h, parts, weight, y, eps=EPS, fm=False):
 
 # ---- fragment-major operands (include/wptv.h) and the products that read them ----
 
-FM_MAX_ROWS = 320  # rows the fm products take (up to 160, or 289 to 320)
+FM_MAX_ROWS = 320  # rows the fm products take (up to 160, or 289 to 320; any_rows: 161 to 288 too)
 
 
 def _same(y, h):
@@ -371,30 +371,35 @@ class FmWeight:
         self.data = fm_pack(w.contiguous(), w.shape[0] // 16)
 
 
-def fm_plan(M, N, K, swiglu=False):
+def fm_plan(M, N, K, swiglu=False, any_rows=False):
     """(parts, parts bytes) of an fm product, or None where no kernel form
-    takes the shape."""
+    takes the shape.  any_rows: the products of 161 to 288 rows included
+    (wptv_gemm_fm_any_*)."""
     if not 0 < M <= FM_MAX_ROWS:
         return None
     parts = _lib.ctypes.c_int(1 if swiglu else 0)
     size = _lib.ctypes.c_size_t(0)
-    status = _lib.lib().wptv_gemm_fm_plan(M, N, K, int(swiglu), _lib.ctypes.byref(parts), _lib.ctypes.byref(size))
+    plan = _lib.lib().wptv_gemm_fm_any_plan if any_rows else _lib.lib().wptv_gemm_fm_plan
+    status = plan(M, N, K, int(swiglu), _lib.ctypes.byref(parts), _lib.ctypes.byref(size))
     return (parts.value, size.value) if status == 0 else None
 
 
-def linear_fm_parts(x_fm, rows, w, splits=0):
+def linear_fm_parts(x_fm, rows, w, splits=0, any_rows=False):
     """The split-K parts (S, rows, N) FP32 of x . w^T, x a flat fm operand of
-    rows x K, w an FmWeight (N, K) (wptv_gemm_fm_parts)."""
+    rows x K, w an FmWeight (N, K) (wptv_gemm_fm_parts; any_rows:
+    wptv_gemm_fm_any_parts)."""
     _gpu(x_fm, w.data)
     N, K = w.shape
     _fm_output(x_fm, rows, K)
     library = _lib.lib()
     parts = _lib.ctypes.c_int(int(splits))
     size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_gemm_fm_plan(rows, N, K, 0, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm_fm")
+    plan, product = ((library.wptv_gemm_fm_any_plan, library.wptv_gemm_fm_any_parts) if any_rows else
+                     (library.wptv_gemm_fm_plan, library.wptv_gemm_fm_parts))
+    check(plan(rows, N, K, 0, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm_fm")
     out = torch.empty(parts.value, rows, N, dtype=torch.float32, device=x_fm.device)
-    check(library.wptv_gemm_fm_parts(ptr(x_fm), ptr(w.data), rows, N, K, parts.value, ptr(out), out.numel() * 4,
-                                     _lib.stream(x_fm.device)), "gemm_fm_parts")
+    check(product(ptr(x_fm), ptr(w.data), rows, N, K, parts.value, ptr(out), out.numel() * 4,
+                  _lib.stream(x_fm.device)), "gemm_fm_parts")
     return out
 
 
@@ -433,14 +438,15 @@ def head_argmax_fm_wide(x_fm, rows, w):
     return best
 
 
-def linear_fm_swiglu(x_fm, rows, w):
+def linear_fm_swiglu(x_fm, rows, w, any_rows=False):
     """silu(gate) * up of x (a flat fm operand of rows x K) and the gate/up
     FmWeight packed from interleave_gate_up's order: a flat fm operand of
-    rows x N / 2, the down product's X (wptv_gemm_fm_swiglu)."""
+    rows x N / 2, the down product's X (wptv_gemm_fm_swiglu; any_rows:
+    wptv_gemm_fm_any_swiglu)."""
     _gpu(x_fm, w.data)
     N, K = w.shape
     _fm_output(x_fm, rows, K)
     out = fm_empty(rows, N // 2, x_fm.device)
-    check(_lib.lib().wptv_gemm_fm_swiglu(ptr(x_fm), ptr(w.data), rows, N, K, ptr(out), _lib.stream(x_fm.device)),
-          "gemm_fm_swiglu")
+    product = _lib.lib().wptv_gemm_fm_any_swiglu if any_rows else _lib.lib().wptv_gemm_fm_swiglu
+    check(product(ptr(x_fm), ptr(w.data), rows, N, K, ptr(out), _lib.stream(x_fm.device)), "gemm_fm_swiglu")
     return out
