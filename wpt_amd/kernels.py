@@ -50,8 +50,10 @@ class _ForwardOnly(torch.autograd.Function):
 
 
 def _forward_only(out, *inputs):
-    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in inputs):
-        return _ForwardOnly.apply(out, *[x for x in inputs if x is not None])
+    if torch.is_grad_enabled():
+        for x in inputs:
+            if x is not None and x.requires_grad:
+                return _ForwardOnly.apply(out, *[x for x in inputs if x is not None])
     return out
 
 
@@ -60,23 +62,36 @@ def _check_inputs(q, k, v, positions):
         raise ValueError(f"q must be (B, T, H, c) and k, v (B, N, c); got {tuple(q.shape)}, {tuple(k.shape)}, "
                          f"{tuple(v.shape)}")
     B, T, H, c = q.shape
-    if k.shape != v.shape or k.shape[0] != B or k.shape[2] != c:
+    Bk, N, ck = k.shape
+    if k.shape != v.shape or Bk != B or ck != c:
         raise ValueError(f"k and v must be (B={B}, N, c={c}); got {tuple(k.shape)}, {tuple(v.shape)}")
-    if not (q.dtype == k.dtype == v.dtype):
+    dtype, device = q.dtype, q.device
+    if k.dtype != dtype or v.dtype != dtype:
         raise ValueError(f"q, k and v must share one dtype; got {q.dtype}, {k.dtype}, {v.dtype}")
-    if not (q.device == k.device == v.device) or q.device.type != "cuda":
+    if k.device != device or v.device != device or device.type != "cuda":
         raise KernelUnavailable(f"the HIP attention runs on a GPU; q is on {q.device}")
     if k.stride(2) != 1 or v.stride(2) != 1:
         raise ValueError("each row of k and v must be contiguous")
-    if positions is not None and tuple(positions.shape) != (B, T):
+    if positions is not None and positions.shape != (B, T):
         raise ValueError(f"positions must be (B={B}, T={T}); got {tuple(positions.shape)}")
-    if k.shape[1] == 0:
+    if N == 0:
         raise ValueError("the table is empty")
-    return B, T, H, c, k.shape[1]
+    return B, T, H, c, N
 
 
 def _long(x, device):
+    if x.dtype is torch.long and x.device == device and x.is_contiguous():
+        return x
     return x.to(device=device, dtype=torch.long).contiguous()
+
+
+def _sink(sink, H, device):
+    """The sink (H,) as the kernels read it."""
+    if sink.dtype is not torch.float32 or sink.device != device or not sink.is_contiguous():
+        sink = sink.to(device=device, dtype=torch.float32).contiguous()
+    if sink.shape != (H,):
+        raise ValueError(f"sink must be (H={H},); got {tuple(sink.shape)}")
+    return sink
 
 
 def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=None, lse=False, splits=0,
@@ -108,9 +123,7 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
     positions_ = None if positions is None else _long(positions, device)
     if out_fm and (static_scratch or q.dtype != torch.bfloat16):
         raise ValueError("the fm output layout takes bf16 queries and the workspace entry point")
-    sink_ = None if sink is None else sink.to(device=device, dtype=torch.float32).contiguous()
-    if sink_ is not None and sink_.shape != (H,):
-        raise ValueError(f"sink must be (H={H},); got {tuple(sink_.shape)}")
+    sink_ = None if sink is None else _sink(sink, H, device)
     tree_base = ancestors = None
     if tree is not None:
         tree_base, ancestors = (_long(x, device) for x in tree)
@@ -119,10 +132,8 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
     flags = ((_lib.FORCE_GENERIC if generic else 0) | (_lib.RANGE_FROM_POSITIONS if from_positions else 0)
              | (_lib.KEY_SPLIT if key_split else 0) | (_lib.OUT_FM if out_fm else 0)
              | (_lib.ROWS32 if rows32 else 0))
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_attention_workspace(B, T, H, c, N, int(window), dtype, flags, _lib.ctypes.byref(parts),
-                                           _lib.ctypes.byref(size)), "verify_attention")
+    parts, size = _lib.plan("wptv_attention_workspace", "verify_attention", B, T, H, c, N, int(window), dtype, flags,
+                            splits=int(splits))
     out = torch.empty_like(q_)
     lse_out = torch.empty(B, T, H, dtype=torch.float32, device=device) if lse else None
     if static_scratch:
@@ -133,14 +144,13 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
               "verify_attention_static")
         out = _forward_only(out, q, k, v, sink)
         return (out, lse_out) if lse else out
-    workspace = torch.empty(max(1, size.value), dtype=torch.uint8, device=device) if size.value else None
+    workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
     if out_fm:  # [B T, H c] as the output projection's fm operand (layers.fm_unpack reads it back)
         out = torch.empty(_lib.fm_row_blocks(B * T) * 16 * H * c, dtype=q.dtype, device=device)
     check(library.wptv_verify_attention(ptr(q_), ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1),
                                         dtype, ptr(positions_), int(window), ptr(tree_base), ptr(ancestors),
-                                        ptr(sink_), B, T, H, c, N, float(scale), parts.value, flags, ptr(out),
-                                        ptr(lse_out), ptr(workspace), size.value, _lib.stream(device)),
-          "verify_attention")
+                                        ptr(sink_), B, T, H, c, N, float(scale), parts, flags, ptr(out),
+                                        ptr(lse_out), ptr(workspace), size, _lib.stream(device)), "verify_attention")
     if not out_fm:
         out = _forward_only(out, q, k, v, sink)
     return (out, lse_out) if lse else out
@@ -182,14 +192,13 @@ def choose_rows(q, k, positions, lse, scale, top_k, window):
     if not K:
         return chosen
     library = _lib.lib()
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_choice_workspace(B, T, N, _lib.ctypes.byref(size)), "choose_rows")
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=device)
+    _, size = _lib.plan("wptv_choice_workspace", "choose_rows", B, T, N)
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
     q_ = q.contiguous()
     positions_ = _long(positions, device)
     check(library.wptv_exact_choice(ptr(q_), ptr(k), k.stride(0), k.stride(1), _lib.dtype_code(q.dtype),
                                     ptr(positions_), ptr(lse.contiguous()), B, T, H, c, N, float(scale), int(top_k),
-                                    int(window), ptr(chosen), ptr(workspace), size.value, _lib.stream(device)),
+                                    int(window), ptr(chosen), ptr(workspace), size, _lib.stream(device)),
           "choose_rows")
     return chosen
 
@@ -213,9 +222,7 @@ def sparse_attention(q, k, v, sink, idx, positions, scale, window, *, gate=None,
     q_ = q.contiguous()
     idx_ = _long(idx, device)
     positions_ = _long(positions, device)
-    sink_ = sink.to(device=device, dtype=torch.float32).contiguous()
-    if sink_.shape != (H,):
-        raise ValueError(f"sink must be (H={H},); got {tuple(sink_.shape)}")
+    sink_ = _sink(sink, H, device)
     gate_stride = 0
     if gate is not None:
         if gate.dtype != q.dtype or gate.shape[:2] != (B, T) or gate.stride(-1) != 1 or \
@@ -223,16 +230,14 @@ def sparse_attention(q, k, v, sink, idx, positions, scale, window, *, gate=None,
             raise ValueError(f"gate must be (B={B}, T={T}, >= H*c) in q's dtype, rows one after another")
         gate_stride = gate.stride(1)
     K = idx_.shape[2]
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_sparse_attention_workspace(B, T, H, c, K, int(window), N, dtype, _lib.ctypes.byref(parts),
-                                                  _lib.ctypes.byref(size)), "sparse_attention")
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=device) if size.value else None
+    parts, size = _lib.plan("wptv_sparse_attention_workspace", "sparse_attention", B, T, H, c, K, int(window), N, dtype,
+                            splits=int(splits))
+    workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
     out = torch.empty_like(q_)
     check(library.wptv_sparse_attention(ptr(q_), ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1),
                                         dtype, ptr(idx_), K, ptr(positions_), int(window), ptr(sink_), ptr(gate),
-                                        gate_stride, B, T, H, c, N, float(scale), parts.value, ptr(out), None,
-                                        ptr(workspace), size.value, _lib.stream(device)), "sparse_attention")
+                                        gate_stride, B, T, H, c, N, float(scale), parts, ptr(out), None,
+                                        ptr(workspace), size, _lib.stream(device)), "sparse_attention")
     return _forward_only(out, q, k, v, sink)
 
 
@@ -246,10 +251,8 @@ def _window_call(q, k, v, sink, positions, scale, window, row_base, ring_rows, g
         raise KernelUnavailable(f"the HIP window attention runs on a GPU; q is on {q.device}")
     if k.stride(2) != 1 or v.stride(2) != 1:
         raise ValueError("each row of k and v must be contiguous")
-    if sink.shape != (H,):
-        raise ValueError(f"sink must be (H={H},); got {tuple(sink.shape)}")
+    sink_ = _sink(sink, H, device)
     positions_ = _long(positions.expand(B, T), device)
-    sink_ = sink.to(device=device, dtype=torch.float32).contiguous()
     gate_stride = 0
     if gate is not None:
         if gate.dtype != q.dtype or gate.shape[:2] != (B, T) or gate.stride(-1) != 1 or \
@@ -258,17 +261,15 @@ def _window_call(q, k, v, sink, positions, scale, window, row_base, ring_rows, g
         gate_stride = gate.stride(1)
     library = _lib.lib()
     dtype = _lib.dtype_code(q.dtype)
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_window_attention_workspace(B, T, H, c, int(window), dtype, _lib.ctypes.byref(parts),
-                                                  _lib.ctypes.byref(size)), "window_attention")
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=device) if size.value else None
+    parts, size = _lib.plan("wptv_window_attention_workspace", "window_attention", B, T, H, c, int(window), dtype,
+                            splits=int(splits))
+    workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
     q_ = q.contiguous()
     out = torch.empty_like(q_)
     check(library.wptv_window_attention(ptr(q_), ptr(k), k.stride(0), k.stride(1), ptr(v), v.stride(0), v.stride(1),
                                         dtype, ptr(positions_), ptr(row_base), int(ring_rows), int(window), ptr(sink_),
-                                        ptr(gate), gate_stride, B, T, H, c, float(scale), parts.value, ptr(out),
-                                        ptr(workspace), size.value, _lib.stream(device)), "window_attention")
+                                        ptr(gate), gate_stride, B, T, H, c, float(scale), parts, ptr(out),
+                                        ptr(workspace), size, _lib.stream(device)), "window_attention")
     return _forward_only(out, q, k, v, sink)
 
 

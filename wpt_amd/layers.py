@@ -204,15 +204,13 @@ def linear(x, w, out_dtype=None, splits=0):
     M = x2.shape[0]
     out_dtype = torch.bfloat16 if out_dtype is None else out_dtype
     code = _lib.dtype_code(out_dtype)
-    library = _lib.lib()
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
+    parts, size = int(splits), 0
     if not (splits == 0 and wide_tiles(M, N, K)):  # the wide tiles need no split count and no workspace
-        check(library.wptv_gemm_workspace(M, N, K, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm")
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=x.device) if size.value else None
+        parts, size = _lib.plan("wptv_gemm_workspace", "gemm", M, N, K, splits=int(splits))
+    workspace = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
     out = torch.empty(M, N, dtype=out_dtype, device=x.device)
-    check(library.wptv_gemm(ptr(x2), x2.stride(0), ptr(w), w.stride(0), M, N, K, ptr(out), out.stride(0), code,
-                            parts.value, ptr(workspace), size.value, _lib.stream(x.device)), "gemm")
+    check(_lib.lib().wptv_gemm(ptr(x2), x2.stride(0), ptr(w), w.stride(0), M, N, K, ptr(out), out.stride(0), code,
+                               parts, ptr(workspace), size, _lib.stream(x.device)), "gemm")
     return out.reshape(*x.shape[:-1], N)
 
 
@@ -285,16 +283,12 @@ def linear_parts(x, w, splits=0, max_splits=8):
     if x2.stride(1) != 1:
         x2 = x2.contiguous()
     M = x2.shape[0]
-    library = _lib.lib()
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_gemm_workspace(M, N, K, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm_parts")
-    if parts.value > max_splits:
-        parts = _lib.ctypes.c_int(int(max_splits))
-        check(library.wptv_gemm_workspace(M, N, K, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm_parts")
-    out = torch.empty(parts.value, M, N, dtype=torch.float32, device=x.device)
-    check(library.wptv_gemm_parts(ptr(x2), x2.stride(0), ptr(w), w.stride(0), M, N, K, parts.value, ptr(out),
-                                  out.numel() * 4, _lib.stream(x.device)), "gemm_parts")
+    parts, _ = _lib.plan("wptv_gemm_workspace", "gemm_parts", M, N, K, splits=int(splits))
+    if parts > max_splits:
+        parts, _ = _lib.plan("wptv_gemm_workspace", "gemm_parts", M, N, K, splits=int(max_splits))
+    out = torch.empty(parts, M, N, dtype=torch.float32, device=x.device)
+    check(_lib.lib().wptv_gemm_parts(ptr(x2), x2.stride(0), ptr(w), w.stride(0), M, N, K, parts, ptr(out),
+                                     out.numel() * 4, _lib.stream(x.device)), "gemm_parts")
     return out
 
 
@@ -392,14 +386,12 @@ def linear_fm_parts(x_fm, rows, w, splits=0, any_rows=False):
     N, K = w.shape
     _fm_output(x_fm, rows, K)
     library = _lib.lib()
-    parts = _lib.ctypes.c_int(int(splits))
-    size = _lib.ctypes.c_size_t(0)
-    plan, product = ((library.wptv_gemm_fm_any_plan, library.wptv_gemm_fm_any_parts) if any_rows else
-                     (library.wptv_gemm_fm_plan, library.wptv_gemm_fm_parts))
-    check(plan(rows, N, K, 0, _lib.ctypes.byref(parts), _lib.ctypes.byref(size)), "gemm_fm")
-    out = torch.empty(parts.value, rows, N, dtype=torch.float32, device=x_fm.device)
-    check(product(ptr(x_fm), ptr(w.data), rows, N, K, parts.value, ptr(out), out.numel() * 4,
-                  _lib.stream(x_fm.device)), "gemm_fm_parts")
+    plan, product = (("wptv_gemm_fm_any_plan", library.wptv_gemm_fm_any_parts) if any_rows else
+                     ("wptv_gemm_fm_plan", library.wptv_gemm_fm_parts))
+    parts, _ = _lib.plan(plan, "gemm_fm", rows, N, K, 0, splits=int(splits))
+    out = torch.empty(parts, rows, N, dtype=torch.float32, device=x_fm.device)
+    check(product(ptr(x_fm), ptr(w.data), rows, N, K, parts, ptr(out), out.numel() * 4, _lib.stream(x_fm.device)),
+          "gemm_fm_parts")
     return out
 
 
@@ -428,13 +420,11 @@ def head_argmax_fm_wide(x_fm, rows, w):
     N, K = w.shape
     _fm_output(x_fm, rows, K)
     blocks = x_fm.numel() // (16 * K)
-    library = _lib.lib()
-    size = _lib.ctypes.c_size_t(0)
-    check(library.wptv_gemm_fm_wide_argmax_workspace(rows, N, _lib.ctypes.byref(size)), "gemm_fm_wide_argmax")
-    workspace = torch.empty(size.value, dtype=torch.uint8, device=x_fm.device)
+    _, size = _lib.plan("wptv_gemm_fm_wide_argmax_workspace", "gemm_fm_wide_argmax", rows, N)
+    workspace = torch.empty(size, dtype=torch.uint8, device=x_fm.device)
     best = torch.empty(rows, dtype=torch.int32, device=x_fm.device)
-    check(library.wptv_gemm_fm_wide_argmax(ptr(x_fm), blocks, ptr(w.data), rows, N, K, ptr(best), ptr(workspace),
-                                           size.value, _lib.stream(x_fm.device)), "gemm_fm_wide_argmax")
+    check(_lib.lib().wptv_gemm_fm_wide_argmax(ptr(x_fm), blocks, ptr(w.data), rows, N, K, ptr(best), ptr(workspace),
+                                              size, _lib.stream(x_fm.device)), "gemm_fm_wide_argmax")
     return best
 
 

@@ -54,9 +54,8 @@ def _scores(x):
 
 
 def _workspace(device, B, L):
-    size = _lib.ctypes.c_size_t(0)
-    check(_lib.lib().wptv_accept_workspace(B, L, _lib.ctypes.byref(size)), "accept")
-    return torch.empty(size.value, dtype=torch.uint8, device=device), size.value
+    _, size = _lib.plan("wptv_accept_workspace", "accept", B, L)
+    return torch.empty(size, dtype=torch.uint8, device=device), size
 
 
 def draws(B, L, V, generator=None, device="cuda"):
@@ -89,6 +88,10 @@ def _inputs(scores, q, drafts, lengths, firsts, greedy, temperature):
             raise ValueError(f"the temperature must be positive; got {temperature}")
     else:
         q = None
+    if lengths is None and firsts is None:  # every row: L drafts from its first position
+        if scores.shape[1] < L + 1:
+            raise ValueError(f"scores hold {scores.shape[1]} positions per row; {L + 1} are read")
+        return (scores, q, drafts, None, None), (B, L, V)
     lengths_ = None if lengths is None else torch.as_tensor(lengths, dtype=torch.int32, device=device).contiguous()
     firsts_ = None if firsts is None else torch.as_tensor(firsts, dtype=torch.int32, device=device).contiguous()
     host_lengths = torch.full((B,), L) if lengths is None else torch.as_tensor(lengths).cpu().long()
