@@ -408,3 +408,35 @@ def test_the_fused_commit_equals_accept_undo_and_next_feeds(device, greedy, top_
         assert int(c2[0]) == -1 and int(fused[4]) == 1
         assert int(fused[0][0]) == int(before[0]) and torch.equal(fused[2][0].cpu(), feeds[0])
     assert int(fused[0][1]) <= int(before[1]) + 2
+
+
+@pytest.mark.parametrize("B, L, V, top_k, kind", [
+    (3, 4, 32768, 40, "spread"), (2, 2, 32768, 128, "spread"), (9, 1, 4096, 1, "spread"), (2, 3, 131, 128, "spread"),
+    (2, 2, 32768, 40, "one thread"), (2, 2, 8192, 40, "ties"), (1, 2, 50001, 100, "spread"), (2, 2, 30011, 7, "few"),
+    (2, 2, 4096, 40, "equal")])
+def test_a_small_cut_decides_as_the_full_rows_do(device, B, L, V, top_k, kind):
+    # the kept entries alone against the oracle on the same tape: entries past
+    # the row, all kept entries in one thread (a wavefront walks), ties at the
+    # cut, more entries at the floor than the list holds, rows of -inf but for
+    # fewer than top_k entries
+    g = torch.Generator().manual_seed(B * V + top_k)
+    scores = 3 * torch.randn(B, L + 1, V, generator=g)
+    if kind == "one thread":
+        scores[..., 5::1024] += 20.0
+    elif kind == "ties":
+        scores = scores.round()
+    elif kind == "few":
+        kept = torch.zeros(V, dtype=torch.bool)
+        kept[torch.randperm(V, generator=g)[:3]] = True
+        scores = scores.masked_fill(~kept, -float("inf"))
+    elif kind == "equal":
+        scores[:] = 1.5
+    q = torch.softmax(scores[:, :L].nan_to_num(neginf=-50.0) + 0.5 * torch.randn(B, L, V, generator=g), -1)
+    drafts = torch.multinomial(q.reshape(B * L, V), 1, generator=g).reshape(B, L)
+    u = torch.rand(B, L, generator=g)
+    e = torch.empty(B, V).exponential_(generator=g)
+    lengths = [L] * B
+    expected = oracle.accept(scores, q, drafts, lengths, 0.7, top_k, [oracle.TapeDraws(u[b], e[b]) for b in range(B)])
+    tokens, counts = sampling.accept(*(x.to(device) for x in (scores, q, drafts, u, e)), 0.7, top_k)
+    got = sampling.written(tokens, counts)
+    assert not compare(got, expected, oracle.margins(scores, q, drafts, lengths, 0.7, top_k, u))

@@ -15,6 +15,8 @@
 //                  draw from a distribution by the exponential race torch's
 //                  multinomial uses); in greedy mode the first maximal index
 //                  instead, the draft kept iff it is that index
+//   accept_stats_cut  the same with a small top-k cut: only the kept entries
+//                  have a p, so only their exponentials and draft entries are read
 //   accept_pick    one thread per batch row: the first rejected draft and the
 //                  row's tokens from the per-position results
 //   tree_walk      greedy verification of a draft tree from the per-node argmax
@@ -549,6 +551,250 @@ __global__ __launch_bounds__(kT) void accept_stats(const S* __restrict__ scores,
   }
 }
 
+// With a top-k cut of at most kQuickK entries.  Only the kept entries (the k largest and
+// the ties with the k-th) have a p, so only they are exponentiated, and of the
+// draft and exponential rows only their entries are read (a draft distribution
+// is nowhere negative: an entry with p = 0 leaves max(0, p - q) = 0).  A
+// thread holds at most two kept entries as a rule, in slots; a wavefront with a
+// thread of more walks its entries.  Every sum adds the same values in the same
+// order as over the whole row, the zeros left out.
+//
+// The k-th largest: each wavefront finds the r-th largest of its
+// threads' own maxima, r = ceil(k / 16), by bits of a ballot (the low 16 bits
+// left 0: a lower bound serves); the least of those is a floor that at least
+// 16 r >= k entries reach.  The entries at or above it (some hundred) are
+// gathered in LDS and each counts the ones above it.  Four barriers, where the
+// radix select (kth_largest: here only if more than kT reach the floor) takes 26.
+//
+// Measured on the MI355X at batch 32, 4 drafts, 32768 entries, bf16 scores, graph
+// replays of both launches, accept_stats then this, us: k = 5 29.4, 18.4; 40
+// 32.2, 21.4 (in order 38.3, 33.3; FP32 scores 34.1, 21.3); 128 32.6, 26.7; 200
+// 33.2, 30.4 but in order 40.8, 41.3; 1500 40.3, 48.2: with k past a hundred
+// or two some thread of every wavefront has more than two kept entries.
+constexpr int kQuickK = 128;
+
+template <int ITEMS, typename S, bool ORDER>
+__global__ __launch_bounds__(kT) void accept_stats_cut(const S* __restrict__ scores, int64_t sb, int64_t st,
+                                                       const int32_t* __restrict__ firsts,
+                                                       const float* __restrict__ q, int64_t qb, int64_t qt,
+                                                       const int64_t* __restrict__ drafts, int64_t db,
+                                                       const int32_t* __restrict__ lengths,
+                                                       const float* __restrict__ u, const float* __restrict__ e,
+                                                       float temperature, int top_k, int B, int L, int V,
+                                                       Stats stats) {
+  __shared__ float redv[kW];
+  __shared__ int redi[kW];
+  __shared__ int hist[256];
+  __shared__ int sel[2];
+  __shared__ __attribute__((aligned(16))) uint32_t list[kT + 4];
+  __shared__ int gathered;
+  // a row's positions on one XCD, as accept_stats
+  const int P = L + 1, slot = blockIdx.x >> 3;
+  const int b = 8 * (slot / P) + (blockIdx.x & 7), j = slot % P;
+  if constexpr (ORDER) {  // order_draw, the next launch, counts each row's slices from zero
+    if (blockIdx.x == 0)
+      for (int i = threadIdx.x; i < B; i += kT) stats.arrivals[i] = 0;
+  }
+  if (b >= B) return;
+  const int n = lengths ? min(max(lengths[b], 0), L) : L;
+  if (j > n) return;
+  const int64_t first = firsts ? firsts[b] : 0;
+  const S* row = scores + b * sb + (first + j) * st;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, idx = b * P + j;
+  const bool draft_pos = j < n;
+  const float* qrow = draft_pos ? q + b * qb + j * qt : nullptr;
+  const float* erow = ORDER ? nullptr : e + (int64_t)b * V;
+  S bits[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) bits[i] = score_bits<S>(row, V, i);
+  const int64_t d = draft_pos ? drafts[b * db + j] : -1;
+  // the thread that holds the draft's score
+  const bool in_row = d >= 0 && d < V, owner = in_row && (int)(d & (kT - 1)) == tid;
+  const float qd = owner ? qrow[d] : 0.f;
+  const float ud = !ORDER && owner ? u[(int64_t)b * L + j] : 0.f;
+
+  float x[ITEMS];
+  const float tinv = 1.f / temperature;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) x[i] = div_by(score_value<S>(bits[i]), temperature, tinv);
+  if (V < ITEMS * kT) {  // entries past the row: never among the k < V largest but for ties at -inf, whose p is 0
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+      if (tid + i * kT >= V) x[i] = kNegInfS;
+  }
+  float mx = kNegInfS;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) mx = fmaxf(mx, x[i]);
+
+  float m, thr;
+  bool quick;
+  {
+    const int r = (top_k + kW - 1) / kW;
+    const uint32_t own = order_key(mx);
+    uint32_t reach = 0;  // the largest 16-bit prefix that r of the wavefront's maxima reach
+#pragma unroll
+    for (int bit = 31; bit >= 16; --bit) {
+      const uint32_t next = reach | (1u << bit);
+      if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(own >= next)) >= r) reach = next;
+    }
+    const float wmax = wave_max(mx);
+    if (lane == 0) {
+      redv[wave] = wmax;
+      redi[wave] = (int)reach;
+    }
+    list[tid] = 0;
+    if (tid < 4) list[kT + tid] = 0;
+    if (tid == 0) gathered = 0;
+    __syncthreads();
+    uint32_t floor = 0xffffffffu;
+    m = kNegInfS;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      floor = min(floor, (uint32_t)redi[w]);
+      m = fmaxf(m, redv[w]);
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const uint32_t key = order_key(x[i]);
+      if (__builtin_amdgcn_ballot_w64(key >= floor) == 0) continue;
+      if (key >= floor) {
+        const int at = atomicAdd(&gathered, 1);
+        if (at < kT) list[at] = key;
+      }
+    }
+    __syncthreads();
+    const int count = gathered;
+    quick = count >= top_k && count <= kT;
+    if (quick) {
+      if (tid < count) {
+        const uint32_t mine = list[tid];
+        int above = 0, same = 0;
+        for (int c = 0; c < count; c += 4) {  // past the count: zeros, above no entry
+          const uint4 k4 = *reinterpret_cast<const uint4*>(list + c);
+          above += (k4.x > mine) + (k4.y > mine) + (k4.z > mine) + (k4.w > mine);
+          same += (k4.x == mine) + (k4.y == mine) + (k4.z == mine) + (k4.w == mine);
+        }
+        if (above < top_k && above + same >= top_k) sel[0] = (int)mine;  // every such thread the same
+      }
+      __syncthreads();
+      thr = key_value((uint32_t)sel[0]);
+    }
+  }
+  if (!quick) thr = kth_largest<ITEMS>(x, top_k, hist, sel, redv);
+
+  // this thread's kept entries
+  int kept = 0, i0 = 0, i1 = 0;
+  float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (__builtin_amdgcn_ballot_w64(x[i] >= thr) == 0) continue;
+    if (x[i] >= thr) {
+      if (kept == 0) {
+        i0 = i;
+        p0 = x[i];
+      } else if (kept == 1) {
+        i1 = i;
+        p1 = x[i];
+      }
+      ++kept;
+    }
+  }
+  const bool walk = __builtin_amdgcn_ballot_w64(kept > 2) != 0;  // the same in every lane of the wavefront
+  const int v0 = tid + i0 * kT, v1 = tid + i1 * kT;
+  // an entry past the row is kept only at -inf: its p is 0 and nothing of it is read
+  const bool at0 = kept > 0 && v0 < V, at1 = kept > 1 && v1 < V;
+  const float q0 = draft_pos && at0 ? qrow[v0] : 0.f, q1 = draft_pos && at1 ? qrow[v1] : 0.f;
+  const float e0 = !ORDER && at0 ? erow[v0] : 1.f, e1 = !ORDER && at1 ? erow[v1] : 1.f;
+  float part;
+  if (walk) {
+    part = 0.f;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      x[i] = x[i] >= thr ? exp_nonpos(x[i] - m) : 0.f;
+      part += x[i];
+    }
+  } else {
+    p0 = kept > 0 ? exp_nonpos(p0 - m) : 0.f;
+    p1 = kept > 1 ? exp_nonpos(p1 - m) : 0.f;
+    part = p0 + p1;
+  }
+  const float z = block_sum(part, redv);
+  const float zinv = 1.f / z;
+  float pd = 0.f;  // p of the draft, in its owner
+  if (walk) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) x[i] = x[i] * zinv;
+    if (owner) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i)
+        if (i == (int)(d >> 10)) pd = x[i];
+    }
+  } else {
+    p0 *= zinv;
+    p1 *= zinv;
+    if (owner) pd = kept > 0 && v0 == (int)d ? p0 : kept > 1 && v1 == (int)d ? p1 : 0.f;
+  }
+  float rest_sum = 1.f;  // the residual's mass (1: the bonus draw from p itself)
+  if (draft_pos) {
+    float rest = 0.f;
+    if (walk) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) {
+        x[i] = x[i] > 0.f ? fmaxf(x[i] - qrow[tid + i * kT], 0.f) : 0.f;
+        rest += x[i];
+      }
+    } else {
+      p0 = fmaxf(p0 - q0, 0.f);
+      p1 = fmaxf(p1 - q1, 0.f);
+      rest = p0 + p1;
+    }
+    rest_sum = block_sum(rest, redv);
+  }
+  if constexpr (ORDER) {
+    if (tid == 0) {
+      stats.m[idx] = m;
+      stats.z[idx] = z;
+      stats.thr[idx] = thr;
+      stats.best[idx] = -1;
+      stats.rest[idx] = rest_sum;
+    }
+    if (owner || (tid == 0 && !in_row)) {  // an out-of-range draft is rejected: u * 0 < 0 never holds
+      stats.pd[idx] = pd;
+      stats.qd[idx] = qd;
+    }
+  } else {
+    float cv = kNegInfS;
+    int ci = INT_MAX;
+    const float rinv = 1.f / rest_sum;
+    auto race = [&](float w, float ex, int v) {
+      const float c = (draft_pos ? div_by(w, rest_sum, rinv) : w) / ex;
+      if (c > cv) {
+        cv = c;
+        ci = v;
+      }
+    };
+    if (walk) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i)
+        if (x[i] > 0.f) race(x[i], erow[tid + i * kT], tid + i * kT);
+    } else {
+      if (at0) race(p0, e0, v0);
+      if (at1) race(p1, e1, v1);
+    }
+    const int drawn = block_argmax(cv, ci, redv, redi);
+    if (tid == 0) {
+      stats.m[idx] = m;
+      stats.z[idx] = z;
+      stats.thr[idx] = thr;
+      stats.best[idx] = -1;
+      // a residual with no mass has no draw (the reference's multinomial raises)
+      stats.cand[idx] = (!(draft_pos && !(rest_sum > 0.f)) && drawn >= 0 && drawn < V) ? drawn : -1;
+      if (!in_row) stats.keep[idx] = 0;
+    }
+    if (owner) stats.keep[idx] = ud * qd < pd;
+  }
+}
+
 // ---- the draws of torch's device generator, in the reference's order --------
 //
 // torch draws on the GPU from Philox4x32-10 (Salmon, Moraes, Dror and Shaw,
@@ -1027,6 +1273,17 @@ void launch_stats(int B, hipStream_t stream, const void* scores, int64_t sb, int
   // the draft rows through LDS when every row is 16-byte aligned and fits
   const bool qlds = !greedy && q && V <= 32 * kT && V % 4 == 0 && aligned(q, 16) && qb % 4 == 0 && qt % 4 == 0;
   const bool cut = !greedy && top_k > 0 && top_k < V;
+  // in order and above 32768 entries the full kernel is the faster one (its 64
+  // entries a thread leave this one no registers: 62.6 against 65.5 us at 50257)
+  if (cut && top_k <= kQuickK && !(ORDER && V > 32 * kT)) {
+#define WPTV_STATS(I)                                                                                               \
+  if constexpr (!(ORDER && I > 32))                                                                                 \
+    hipLaunchKernelGGL((accept_stats_cut<I, S, ORDER>), grid, dim3(kT), 0, stream, rows, sb, st, firsts, q, qb, qt, \
+                       drafts, db, lengths, u, e, temperature, top_k, B, L, V, s);
+    WPTV_ITEMS(V, WPTV_STATS)
+#undef WPTV_STATS
+    return;
+  }
 #define WPTV_STATS_Q(I, QL, CU)                                                                                  \
   hipLaunchKernelGGL((accept_stats<I, S, QL, CU, ORDER>), grid, dim3(kT), 0, stream, rows, sb, st, firsts, q, qb,  \
                      qt, drafts, db, lengths, u, e, temperature, top_k, greedy, B, L, V, s)
