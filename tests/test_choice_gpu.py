@@ -113,3 +113,58 @@ def test_a_bad_lse_is_a_value_error(device):
     with pytest.raises(ValueError):
         kernels.choose_rows(q.to(device), k.to(device), positions.to(device), torch.zeros(1, 4, 3, device=device),
                             0.1, 10, 4)
+
+
+@pytest.mark.parametrize("H, c, T, N, window", [
+    (16, 128, 1, 257, 4), (16, 64, 3, 300, 16), (16, 128, 8, 511, 128), (16, 128, 9, 400, 4), (16, 64, 6, 1030, 1),
+    (8, 128, 1, 64, 4), (8, 64, 3, 255, 16), (8, 128, 7, 770, 128), (8, 128, 16, 513, 0), (8, 64, 17, 300, 16),
+])
+def test_the_scores_of_blocks_of_heads_match_the_formula(device, H, c, T, N, window):
+    # the block kernels' edges: part blocks of positions (8 heads: two a block), table rows past the
+    # last whole batch of 64, the widest reading of the register form and one past it.  FP32 sums of bf16
+    # products: a row may change places with another within 1e-2 of it
+    q, k, _, _, positions = inputs(B=3, T=T, H=H, c=c, N=N, seed=11, dtype=torch.bfloat16)
+    score = choice_scores(q, k, positions, c ** -0.5, window)
+    s = torch.einsum("bthc,bnc->bthn", q.double(), k.double()) * c ** -0.5
+    lse = s.masked_fill(torch.arange(N) > positions[:, :, None, None], float("-inf")).logsumexp(-1).float()
+    K = N // 3
+    rows = kernels.choose_rows(*[x.to(device) for x in (q, k, positions, lse)], c ** -0.5, K, window).cpu()
+    expected = score.topk(min(K, N - window), -1)
+    check_choice(rows, expected.indices.masked_fill(expected.values == float("-inf"), -1), score, 1e-2)
+
+
+def _values(kind, N, generator):
+    if kind == "spread":
+        return torch.randperm(N, generator=generator).float() - N // 2
+    if kind == "equal":
+        return torch.full((N,), 3.0)
+    if kind == "few values":  # far more equal keys than are ranked one by one
+        return torch.randint(3, (N,), generator=generator).float()
+    # one huge value: the rest share the first histogram's lowest bins, or one of them
+    x = torch.randperm(N, generator=generator).float() + 1
+    x[N // 2] = 2.0 ** 100
+    x[N // 3] = -2.0 ** 100
+    return x
+
+
+@pytest.mark.parametrize("kind", ["spread", "equal", "few values", "outliers"])
+@pytest.mark.parametrize("N", [5, 1024, 1025, 2048, 2051, 4096, 4100, 8192, 8197])
+def test_the_select_s_rows_are_a_stable_sort_s(device, kind, N):
+    # one head of width 4 whose first element is the row's value and no log-sum-exp: the order of the
+    # scores is the values' own, equal for equal values, so the rows are known exactly
+    x = _values(kind, N, torch.Generator().manual_seed(N))
+    k = torch.zeros(1, N, 4)
+    k[0, :, 0] = x
+    window = 2
+    q = torch.zeros(1, 2, 1, 4)
+    q[..., 0] = 1.0
+    positions = torch.tensor([[N - 1, N // 2]])
+    for K in sorted({1, max(1, N // 4), max(1, N - window - 1)}):
+        rows = kernels.choose_rows(*[t.to(device) for t in (q, k, positions, torch.zeros(1, 2, 1))], 1.0, K, window)
+        for t, far in enumerate((N - window, N // 2 - window + 1)):
+            order = torch.argsort(x[:far], descending=True, stable=True)[:K]
+            kth = x[order[-1]]
+            want = sorted(r for r in order.tolist() if x[r] > kth) + sorted(r for r in order.tolist() if x[r] == kth)
+            if far <= K:
+                want = list(range(far))
+            assert rows[0, t].tolist() == want + [-1] * (K - len(want)), (kind, N, K, t)

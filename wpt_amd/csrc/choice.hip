@@ -21,14 +21,14 @@
 //                    64 table rows): the scores of the 64 rows for every
 //                    query of the block, written once (4 bytes per row and
 //                    query, against the 2c bytes of the key read once)
-//                      bf16, head width 64 or 128: S^T = K . Q^T on
-//                        v_mfma_f32_16x16x32_bf16 (one key row per lane as
-//                        the A operand), the max over heads through LDS
+//                      bf16, head width 64 or 128: v_mfma_f32_16x16x32_bf16,
+//                        the max over 8 or 16 heads in registers, over other
+//                        counts through LDS
 //                      otherwise: FP32 dot products on the VALU
 //   choice_select_regs  one workgroup per query, tables up to 8192 rows: the
-//                    query's scores in registers, the K-th largest found two
-//                    bits at a time with packed workgroup counts, the chosen
-//                    rows written in row order after one exclusive scan
+//                    query's scores in registers, the K-th largest found by
+//                    a histogram of their range and ranks within its bin, the
+//                    chosen rows written in row order after one scan
 //   choice_select    longer tables: a 4-pass radix select of the K-th
 //                    largest score (order-preserving keys, most significant
 //                    byte first; the scores stay in L2), then one pass that
@@ -138,72 +138,89 @@ __global__ __launch_bounds__(kST) void choice_scores_mfma(
   store_scores(xs, blk, pos_b, T, H, N, window, scores, ns);
 }
 
-// 16 heads (each position's heads are one 16-row MFMA block, so the max over
-// the heads is a reduction over the 16 lanes of a lane group): one
-// workgroup per (batch row, 512 table rows), every position of the pass.
-// Each wavefront takes 128 rows in sub-blocks of 16, the keys of four
-// sub-blocks loaded before the first is used, the queries held in
-// registers for the whole range.
-constexpr int kH16Rows = 512;  // table rows per workgroup
-constexpr int kH16Batch = 4;   // 16-row sub-blocks whose keys are in flight together
+// 8 or 16 heads: the (position, head) query rows in 16-row MFMA blocks (two
+// positions a block at 8 heads), one workgroup per (batch row, 256 table rows),
+// every position of the pass.  A wavefront takes four 16-row sub-blocks with
+// all its keys and queries requested before the first product: one memory round
+// trip, which is what bounds it.  The queries are the A operand, so a lane ends
+// with four heads of one key: their maximum takes three instructions, and the
+// permlane swaps that finish it across the lane groups take the four sub-blocks
+// together, leaving sub-block g in lane group g: 64 consecutive rows a store.
+// Batch 32, 5 queries of 16 heads, 4100 rows: 16.4 us (2.1 TB/s of keys), 18.1
+// with 128 rows a wavefront; 24.0 with the keys as A (16 DPP steps a sub-block
+// and position for the maximum) and two round trips of 64 rows; 8 heads 12.3.
+constexpr int kBlockRows = 256;  // table rows per workgroup
 
-template <int C, int TT>
-__global__ __launch_bounds__(kST) void choice_scores_h16(
+template <int C, int H, int QB>
+__global__ __launch_bounds__(kST) void choice_scores_blocks(
     const unsigned short* __restrict__ q, const unsigned short* __restrict__ k, int64_t ksb, int64_t ksn,
     const int64_t* __restrict__ positions, const float* __restrict__ lse, int T, int N, int window, float scale_log2,
     int nkb, float* __restrict__ scores, int64_t ns) {
+  static_assert(H == 8 || H == 16, "a lane group holds four heads of one position");
   constexpr int S = C / 32;
+  constexpr int kPer = 16 / H;  // positions of a block
   const int b = blockIdx.x / nkb;
-  const int n0 = (blockIdx.x % nkb) * kH16Rows;
+  const int n0 = (blockIdx.x % nkb) * kBlockRows;
   const int64_t* pos_b = positions + (int64_t)b * T;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int wn0 = n0 + 64 * w;
+  const int R = T * H, blocks = (R + 15) / 16;
+  const unsigned short* kb = k + (int64_t)b * ksb;
+  bf16x8 kop[4][S];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    int n = wn0 + 16 * u + j;
+    n = n < N ? n : N - 1;  // clamped rows are not written
+#pragma unroll
+    for (int s = 0; s < S; ++s) kop[u][s] = *reinterpret_cast<const bf16x8*>(kb + (int64_t)n * ksn + 32 * s + 8 * g);
+  }
+  bf16x8 qop[QB][S];
+  float l2[QB][4];
+#pragma unroll
+  for (int t = 0; t < QB; ++t) {
+    const int row = min(16 * t + j, R - 1);  // padding rows repeat the last; their scores are not written
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      qop[t][s] = *reinterpret_cast<const bf16x8*>(q + ((int64_t)b * R + row) * C + 32 * s + 8 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l2[t][i] = lse[(int64_t)b * R + min(16 * t + 4 * g + i, R - 1)] * kLog2e;
+  }
   int far = 0;
   for (int t = 0; t < T; ++t) far = max(far, far_rows(pos_b[t], window, N));
-  if (n0 >= far) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int j = lane & 15, g = lane >> 4;
-  bf16x8 qop[TT][S];
-  float l2[TT];
-  int64_t lim[TT];  // row n is a candidate of position t iff n <= lim[t]
+  if (wn0 >= far) return;
+  const int n = wn0 + lane;
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const int tt = t < T ? t : T - 1;
-    const unsigned short* qrow = q + (((int64_t)b * T + tt) * 16 + j) * C;
+  for (int t = 0; t < QB; ++t) {
+    if (t >= blocks) break;
+    float x[4];
 #pragma unroll
-    for (int s = 0; s < S; ++s) qop[t][s] = *reinterpret_cast<const bf16x8*>(qrow + 32 * s + 8 * g);
-    l2[t] = lse[((int64_t)b * T + tt) * 16 + j] * kLog2e;
-    lim[t] = pos_b[tt] - window;
-  }
-  const int wn0 = n0 + w * (kH16Rows / 4);
-  const unsigned short* kb = k + (int64_t)b * ksb;
-#pragma unroll 1
-  for (int sb0 = 0; sb0 < kH16Rows / 4 / 16; sb0 += kH16Batch) {
-    if (wn0 + 16 * sb0 >= far) break;
-    bf16x8 kop[kH16Batch][S];
+    for (int u = 0; u < 4; ++u) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < kH16Batch; ++u) {
-      int n = wn0 + 16 * (sb0 + u) + j;
-      n = n < N ? n : N - 1;  // clamped rows are not written
+      for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qop[t][s], kop[u][s], acc, 0, 0, 0);
+      // acc[i] = S[query row 16 t + 4 g + i][key 16 u + j]
+      float y[4];
 #pragma unroll
-      for (int s = 0; s < S; ++s) kop[u][s] = *reinterpret_cast<const bf16x8*>(kb + (int64_t)n * ksn + 32 * s + 8 * g);
+      for (int i = 0; i < 4; ++i) y[i] = fmaf(acc[i], scale_log2, -l2[t][i]);
+      x[u] = fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3]));
     }
+    // rows of 16 lanes: z01 = sub-blocks (0, 1, 0, 1), z23 = (2, 3, 2, 3), over lane groups
+    // 0, 1 in the lower half and 2, 3 in the upper; then lo = sub-blocks 0 .. 3 over groups
+    // 0, 1 (8 heads: the block's first position), hi over groups 2, 3 (its second)
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[0]), __float_as_uint(x[1]), false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[2]), __float_as_uint(x[3]), false, false);
+    const float z01 = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const float z23 = fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
+    const auto d = __builtin_amdgcn_permlane32_swap(__float_as_uint(z01), __float_as_uint(z23), false, false);
+    const float lo = __uint_as_float(d[0]), hi = __uint_as_float(d[1]);
+    if (n < N) {
 #pragma unroll
-    for (int u = 0; u < kH16Batch; ++u) {
-      const int nb = wn0 + 16 * (sb0 + u);  // the sub-block's first row
-#pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        if (t >= T) break;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[u][s], qop[t][s], acc, 0, 0, 0);
-        // acc[i] = S^T[row nb + 4g + i][head j]; the max over the 16 heads
-        float x[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = row16_max(fmaf(acc[i], scale_log2, -l2[t]));
-        // lane j < 4 writes row nb + 4g + j: 16 consecutive rows per sub-block
-        const int n = nb + 4 * g + j;
-        if (j < 4 && n < N) {
-          const float v = j == 0 ? x[0] : j == 1 ? x[1] : j == 2 ? x[2] : x[3];
-          scores[((int64_t)b * T + t) * ns + n] = (int64_t)n <= lim[t] ? v : -kInf;
+      for (int e = 0; e < kPer; ++e) {
+        const int tt = kPer * t + e;
+        if (tt < T) {
+          const float v = kPer == 1 ? fmaxf(lo, hi) : e == 0 ? lo : hi;
+          scores[((int64_t)b * T + tt) * ns + n] = n < far_rows(pos_b[tt], window, N) ? v : -kInf;
         }
       }
     }
@@ -335,107 +352,183 @@ __global__ __launch_bounds__(kST) void choice_select(const float* __restrict__ s
   }
 }
 
-// Sum over the workgroup, one barrier: red holds two buffers of one value per
-// wavefront, used in turn (a wavefront writes a round's buffer only after
-// every wavefront has passed the barrier of the round before, and so has read
-// the buffer of two rounds before).
-__device__ __forceinline__ uint64_t block_sum_u64(uint32_t lo, uint32_t hi, uint64_t (*red)[kST / 64], int round) {
-  const uint64_t x = (uint64_t)wave_sum_u32(lo) | ((uint64_t)wave_sum_u32(hi) << 32);
-  if ((threadIdx.x & 63) == 0) red[round & 1][threadIdx.x >> 6] = x;
-  __syncthreads();
-  uint64_t r = 0;
-#pragma unroll
-  for (int i = 0; i < kST / 64; ++i) r += red[round & 1][i];
-  return r;
+// The sum over the lanes up to and including this one; every lane must be
+// active (DPP: shifts within the rows of 16, then the rows' totals carried on).
+__device__ __forceinline__ int wave_scan_i32(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return x;
 }
 
-// The select for up to kST * ITEMS candidates: thread t holds the keys of
-// rows ITEMS t .. ITEMS t + ITEMS - 1 in registers (one memory round trip);
-// the K-th largest key is found two bits at a time from the top (16 rounds,
-// each counting the keys at or above three candidates in one packed
-// reduction), and the chosen rows are written in row order after one
-// exclusive scan of the threads' counts.
-template <int ITEMS>
-__global__ __launch_bounds__(kST) void choice_select_regs(const float* __restrict__ scores, int64_t ns,
-                                                          const int64_t* __restrict__ positions, int N, int window,
-                                                          int K, int64_t* __restrict__ chosen) {
-  static_assert(ITEMS % 4 == 0 && kST * ITEMS <= 65535, "packed counts hold 16 bits");
-  __shared__ uint64_t red[2][kST / 64];
-  __shared__ int scan_g[kST / 64], scan_e[kST / 64];
+// The select for up to 4 V THREADS candidates, one workgroup a query: with
+// nv = ceil(candidates / 4 THREADS) quads each, thread t holds the keys of rows
+// 4 nv t .. 4 nv t + 4 nv - 1 in registers (one memory round trip).  The K-th
+// largest key is found by histograms of 1024 equal bins over the range of keys
+// still open (first smallest to largest): the bin that holds it, then, when
+// that holds at most kCand keys, their ranks among each other by counting, else
+// a histogram of the bin's own range.  A range shrinks 2^9 times a pass at the
+// least, so four passes end it whatever the keys are (equal ones end in a bin
+// of width one); scores take one pass and the ranks.  The chosen rows are
+// gathered in LDS in row order, after one scan of the threads' counts, and
+// written out in whole lines.  A serial chain of barriers bounds it: about ten,
+// where finding the key two bits at a time took eighteen, with every key compared
+// three times between each two.  160 queries, 1024 of 3972 rows: 20.0 -> 6.1 us.
+template <int THREADS, int V>
+__global__ __launch_bounds__(THREADS) void choice_select_regs(const float* __restrict__ scores, int64_t ns,
+                                                              const int64_t* __restrict__ positions, int N,
+                                                              int window, int K, int64_t* __restrict__ chosen) {
+  constexpr int kWaves = THREADS / 64, kBins = 1024, kCand = 256;
+  constexpr int kPerLane = kBins / 64;
+  static_assert(4 * V * THREADS < 65536, "packed counts hold 16 bits");
+  static_assert(kBins % THREADS == 0 && kCand <= THREADS, "bins and candidates a thread");
+  __shared__ __attribute__((aligned(16))) int hist[kBins];
+  __shared__ __attribute__((aligned(16))) uint32_t cand[kCand];
+  __shared__ int range[2][kWaves], counts[kWaves], sel[3], ncand;
+  __shared__ uint32_t found;
+  __shared__ int staged[4 * V * THREADS];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t bt = blockIdx.x;
   const int nf = far_rows(positions[bt], window, N);
   int64_t* out = chosen + bt * K;
   if (nf <= K) {  // every candidate, then none
-    for (int i = tid; i < K; i += kST) out[i] = i < nf ? i : -1;
+    for (int i = tid; i < K; i += THREADS) out[i] = i < nf ? i : -1;
     return;
   }
   const float* s = scores + bt * ns;
-  const int base = tid * ITEMS;
-  uint32_t key[ITEMS];  // 0 (below every score's key) past the candidates
+  const int nv = (nf + 4 * THREADS - 1) / (4 * THREADS);  // 1 .. V: nf <= N <= 4 V THREADS
+  const int base = tid * 4 * nv;
+  const int valid = nf - base;  // this thread's items 0 .. valid - 1 are candidates
+  uint32_t key[4 * V];
 #pragma unroll
-  for (int v4 = 0; v4 < ITEMS / 4; ++v4) {
-    const int n = base + 4 * v4;
+  for (int v = 0; v < V; ++v) {
+    if (v >= nv) break;
+    const int n = base + 4 * v;  // a multiple of 4; the scores' row stride is one of 64
     const f32x4 x = n < nf ? *reinterpret_cast<const f32x4*>(s + n) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) key[4 * v4 + e] = n + e < nf ? order_key(x[e]) : 0u;
+    for (int e = 0; e < 4; ++e) key[4 * v + e] = order_key(x[e]);
   }
-  // the largest t with at least K keys >= t: the K-th largest key
-  uint32_t prefix = 0;
-  for (int shift = 30, round = 0; shift >= 0; shift -= 2, ++round) {
-    const uint32_t c1 = prefix | (1u << shift), c2 = prefix | (2u << shift), c3 = prefix | (3u << shift);
-    uint32_t n12 = 0, n3 = 0;
+  auto each = [&](auto&& f) {  // f(item, key) over this thread's candidates
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      n12 += (key[i] >= c1 ? 1u : 0u) + (key[i] >= c2 ? 65536u : 0u);
-      n3 += key[i] >= c3 ? 1u : 0u;
+    for (int v = 0; v < V; ++v) {
+      if (v >= nv) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * v + e < valid) f(4 * v + e, key[4 * v + e]);
     }
-    const uint64_t sum = block_sum_u64(n12, n3, red, round);
-    const int s1 = (int)(sum & 65535), s2 = (int)((sum >> 16) & 65535), s3 = (int)(sum >> 32);
-    prefix = s3 >= K ? c3 : s2 >= K ? c2 : s1 >= K ? c1 : prefix;
-  }
-  const uint32_t tau = prefix;
-  int cg = 0, ce = 0;
+  };
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    cg += key[i] > tau ? 1 : 0;
-    ce += key[i] == tau ? 1 : 0;
-  }
-  // exclusive scan of (cg, ce) over the threads in row order
-  int ig = cg, ie = ce;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int og = __shfl_up(ig, o, 64), oe = __shfl_up(ie, o, 64);
-    if (lane >= o) {
-      ig += og;
-      ie += oe;
-    }
-  }
-  if (lane == 63) {
-    scan_g[w] = ig;
-    scan_e[w] = ie;
+  for (int i = 0; i < kBins / THREADS; ++i) hist[tid + i * THREADS] = 0;
+  if (tid == 0) ncand = 0;
+  int kmin = INT32_MAX, kmax = INT32_MIN;  // as signed, order kept
+  each([&](int, uint32_t x) {
+    const int y = (int)(x ^ 0x80000000u);
+    kmin = min(kmin, y);
+    kmax = max(kmax, y);
+  });
+  kmin = wave_min_i32(kmin);
+  kmax = wave_max_i32(kmax);
+  if (lane == 0) {
+    range[0][w] = kmin;
+    range[1][w] = kmax;
   }
   __syncthreads();
-  int n_gt = 0, pg = ig - cg, pe = ie - ce;
 #pragma unroll
-  for (int i = 0; i < kST / 64; ++i) {
-    n_gt += scan_g[i];
-    if (i < w) {
-      pg += scan_g[i];
-      pe += scan_e[i];
-    }
+  for (int i = 0; i < kWaves; ++i) {
+    kmin = min(kmin, range[0][i]);
+    kmax = max(kmax, range[1][i]);
   }
-  const int need_eq = K - n_gt;
+  uint32_t lo = (uint32_t)kmin ^ 0x80000000u, hi = (uint32_t)kmax ^ 0x80000000u;
+  int remaining = K;  // the key sought is the remaining-th largest of those in lo .. hi
+  uint32_t tau;
+  for (;;) {
+    const uint32_t span = hi - lo;
+    const int shift = span < kBins ? 0 : 22 - __builtin_clz(span);  // span >> shift < kBins
+    each([&](int, uint32_t x) {
+      if (x >= lo && x <= hi) atomicAdd(&hist[(x - lo) >> shift], 1);
+    });
+    __syncthreads();
+    if (w == 0) {
+      // lane l holds bins top - 15 .. top, top = kBins - 1 - 16 l
+      int cnt[kPerLane], total = 0;
+      const int first = kBins - kPerLane * (lane + 1);
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    const int n = base + i;
-    if (key[i] > tau) {
-      out[pg++] = n;
-    } else if (key[i] == tau) {
-      if (pe < need_eq) out[n_gt + pe] = n;
+      for (int e = 0; e < kPerLane; ++e) total += (cnt[e] = hist[first + e]);
+      const int upto = wave_scan_i32(total);
+      if (upto >= remaining && upto - total < remaining) {  // one lane
+        int above = upto - total, bin = first, c = 0;
+#pragma unroll
+        for (int e = kPerLane - 1; e >= 0; --e) {
+          if (c == 0 && above + cnt[e] >= remaining) {
+            bin = first + e;
+            c = cnt[e];
+          }
+          if (c == 0) above += cnt[e];
+        }
+        sel[0] = bin;
+        sel[1] = above;
+        sel[2] = c;
+      }
+    }
+    __syncthreads();
+    const int count = sel[2];
+    remaining -= sel[1];
+    lo += (uint32_t)sel[0] << shift;
+    if (shift == 0) {  // the bin's keys are equal
+      tau = lo;
+      break;
+    }
+    const uint32_t width = (1u << shift) - 1u;
+    if (hi - lo > width) hi = lo + width;
+    if (count <= kCand) {
+      each([&](int, uint32_t x) {
+        if (x >= lo && x <= hi) cand[atomicAdd(&ncand, 1)] = x;
+      });
+      __syncthreads();
+      if (tid < count) {
+        const uint32_t mine = cand[tid];
+        int gt = 0, ge = 0;
+        for (int i = 0; i < count; ++i) {
+          const uint32_t x = cand[i];
+          gt += x > mine ? 1 : 0;
+          ge += x >= mine ? 1 : 0;
+        }
+        if (gt < remaining && ge >= remaining) found = mine;  // the same key from each that writes
+      }
+      __syncthreads();
+      tau = found;
+      break;
+    }
+#pragma unroll
+    for (int i = 0; i < kBins / THREADS; ++i) hist[tid + i * THREADS] = 0;
+    __syncthreads();
+  }
+  // rows above tau and equal to it, each in row order: one scan of both counts
+  int mine = 0;
+  each([&](int, uint32_t x) { mine += x > tau ? 1 : x == tau ? 65536 : 0; });
+  const int upto = wave_scan_i32(mine);
+  if (lane == 63) counts[w] = upto;
+  __syncthreads();
+  int before = upto - mine, n_gt = 0;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    if (i < w) before += counts[i];
+    n_gt += counts[i] & 65535;
+  }
+  int pg = before & 65535, pe = n_gt + (before >> 16);
+  each([&](int i, uint32_t x) {
+    if (x > tau) {
+      staged[pg++] = base + i;
+    } else if (x == tau) {
+      if (pe < K) staged[pe] = base + i;
       ++pe;
     }
-  }
+  });
+  __syncthreads();
+  for (int i = tid; i < K; i += THREADS) out[i] = staged[i];
 }
 
 }  // namespace
@@ -483,22 +576,28 @@ extern "C" int wptv_exact_choice(const void* q, const void* k, int64_t k_stride_
   const float scale_log2 = scale * kLog2e;
   const bool mfma = dtype == WPTV_BF16 && (c == 64 || c == 128) && aligned(q, 16) && aligned(k, 16) &&
                     k_stride_n % 8 == 0 && k_stride_b % 8 == 0;
-  if (mfma && H == 16 && T <= 8) {
+  // up to 128 query rows: the queries of a workgroup fit its registers
+  if (mfma && (H == 8 || H == 16) && T * H <= kMaxRows) {
     const auto* qq = static_cast<const unsigned short*>(q);
     const auto* kk = static_cast<const unsigned short*>(k);
-    const int nkb16 = (N + kH16Rows - 1) / kH16Rows;
-    const int grid16 = B * nkb16;
-#define WPTV_H16(CC, TT)                                                                                           \
-  choice_scores_h16<CC, TT><<<grid16, kST, 0, stream>>>(qq, kk, k_stride_b, k_stride_n, positions, lse, T, N, window, \
-                                                        scale_log2, nkb16, scores, ns)
+    const int blocks = (T * H + 15) / 16;
+    const int nkbb = (N + kBlockRows - 1) / kBlockRows;
+#define WPTV_BLOCKS(CC, HH, QB)                                                                                   \
+  choice_scores_blocks<CC, HH, QB><<<B * nkbb, kST, 0, stream>>>(qq, kk, k_stride_b, k_stride_n, positions, lse, T, \
+                                                                 N, window, scale_log2, nkbb, scores, ns)
+#define WPTV_BLOCKS_Q(CC, HH)                       \
+  (blocks <= 1   ? WPTV_BLOCKS(CC, HH, 1)           \
+   : blocks <= 2 ? WPTV_BLOCKS(CC, HH, 2)           \
+   : blocks <= 3 ? WPTV_BLOCKS(CC, HH, 3)           \
+   : blocks <= 5 ? WPTV_BLOCKS(CC, HH, 5)           \
+                 : WPTV_BLOCKS(CC, HH, 8))
     if (c == 128) {
-      if (T <= 1) WPTV_H16(128, 1); else if (T <= 2) WPTV_H16(128, 2); else if (T <= 4) WPTV_H16(128, 4);
-      else if (T <= 5) WPTV_H16(128, 5); else WPTV_H16(128, 8);
+      if (H == 16) WPTV_BLOCKS_Q(128, 16); else WPTV_BLOCKS_Q(128, 8);
     } else {
-      if (T <= 1) WPTV_H16(64, 1); else if (T <= 2) WPTV_H16(64, 2); else if (T <= 4) WPTV_H16(64, 4);
-      else if (T <= 5) WPTV_H16(64, 5); else WPTV_H16(64, 8);
+      if (H == 16) WPTV_BLOCKS_Q(64, 16); else WPTV_BLOCKS_Q(64, 8);
     }
-#undef WPTV_H16
+#undef WPTV_BLOCKS_Q
+#undef WPTV_BLOCKS
   } else if (mfma) {
     const auto* qq = static_cast<const unsigned short*>(q);
     const auto* kk = static_cast<const unsigned short*>(k);
@@ -521,14 +620,12 @@ extern "C" int wptv_exact_choice(const void* q, const void* k, int64_t k_stride_
   int status = launched("choice_scores");
   if (status != WPTV_OK) return status;
   // the candidates of a query are at most N rows: in registers up to 8192
-  if (N <= kST * 4)
-    choice_select_regs<4><<<B * T, kST, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
-  else if (N <= kST * 8)
-    choice_select_regs<8><<<B * T, kST, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
-  else if (N <= kST * 16)
-    choice_select_regs<16><<<B * T, kST, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
-  else if (N <= kST * 32)
-    choice_select_regs<32><<<B * T, kST, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
+  if (N <= 1024)
+    choice_select_regs<256, 1><<<B * T, 256, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
+  else if (N <= 2048)
+    choice_select_regs<512, 1><<<B * T, 512, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
+  else if (N <= 8192)
+    choice_select_regs<1024, 2><<<B * T, 1024, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
   else
     choice_select<<<B * T, kST, 0, stream>>>(scores, ns, positions, N, window, K, chosen);
   return launched("choice_select");
