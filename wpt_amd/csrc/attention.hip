@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
   const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_address(ring));
   const bool dma_wave = mb < DMAW;
   const int rbase = row_base(rows, b);
-  auto issue = [&](int it) {  // this wavefront's share of the key set's tile of iteration it
+  auto issue = [&](int it) __attribute__((always_inline)) {  // this wavefront's share of the key set's tile of iteration it
     const int tile = kset + it * kKeySets;
     const uint32_t slot = ring_lds + (uint32_t)(it % G::kSlots) * (G::kElems * 2);
 #pragma unroll
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
   const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_address(ring));
   const bool dma_wave = mb < DMAW;
   const int rbase = row_base(rows, b);
-  auto issue = [&](int it) {
+  auto issue = [&](int it) __attribute__((always_inline)) {
     const int tile = kset + it * kKeySets;
     const uint32_t slot = ring_lds + (uint32_t)(it % G::kSlots) * (G::kElems * 2);
 #pragma unroll
