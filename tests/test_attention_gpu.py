@@ -57,6 +57,31 @@ def test_exact_attention_matches_the_oracle(device, B, T, H, c, N, splits, form)
     assert relative_error(got.cpu(), expected) < 1e-2
 
 
+@pytest.mark.parametrize("B, T, H, c, N, window", [
+    (1, 1, 16, 128, 700, 0),     # one 16-row block, in parts
+    (2, 2, 8, 128, 321, 0),      # the first range of more than ten tiles: parts
+    (47, 1, 16, 128, 352, 0),    # five parts a batch row: 235 of 256 compute units
+    (5, 4, 16, 64, 320, 0),      # ten tiles: one part
+    (130, 2, 16, 64, 450, 0),    # more batch rows than half the compute units: parts in two rounds, or none
+    (3, 21, 16, 128, 400, 0),    # three query groups, taken from the last
+    (2, 130, 16, 128, 131, 0),   # a prompt's groups, the last partly padding
+    (7, 9, 16, 128, 500, 128),   # two groups and a window
+])
+def test_the_chosen_parts_match_the_oracle(device, B, T, H, c, N, window):
+    q = draw(B, T, H, c, seed=21)
+    table, k, v = entries_table(B, N, c, seed=22)
+    positions = (N - T + torch.arange(T)).expand(B, T).contiguous()
+    s = (q.double().flatten(1, 2) @ k.double().mT).reshape(B, T, H, N) * c ** -0.5
+    n = torch.arange(N)
+    hidden = (n > positions[..., None]) | ((n <= positions[..., None] - window) if window else False)
+    p = s.masked_fill(hidden[:, :, None], float("-inf")).softmax(-1)
+    expected = (p.flatten(1, 2) @ v.double()).reshape(B, T, H, c)
+    td = table.to(device)
+    got = kernels.verify_attention(q.to(device), td[..., :c], td[..., c:], positions.to(device), c ** -0.5,
+                                   window=window, from_positions=True)
+    assert relative_error(got.cpu(), expected) < 1e-2
+
+
 def test_padding_queries_past_the_table(device):
     # the reference's generation pass: rows at different places, the last
     # row's later queries past the table read up to its last row

@@ -590,7 +590,7 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
 //                               keys, two transposed 4-row reads
 template <int C, int MB, bool TREE>
 __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
-    const int64_t* __restrict__ positions, const int64_t* __restrict__ tree_base, int xcd_map, int groups,
+    const int64_t* __restrict__ positions, const int64_t* __restrict__ tree_base, int B, int groups,
     int splits, int T, int H, int N, int window, int range_from_positions, const unsigned short* __restrict__ k,
     int64_t ksb, int64_t ksn, const unsigned short* __restrict__ v, int64_t vsb, int64_t vsn,
     const unsigned short* __restrict__ q, const uint64_t* __restrict__ ancestors, const float* __restrict__ sink,
@@ -618,24 +618,14 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
   const int j = lane & 31;  // this lane's query row (S^T, O^T columns) or key row (K operand)
   const int h = lane >> 5;  // lane half
 
-  // Workgroups are dealt to the 8 XCDs in turn: every group and split of a
-  // batch row share one XCD (its L2), where several groups read the same
-  // keys and values
-  int unit, split;
-  {
-    const int L = blockIdx.x;
-    if (xcd_map) {
-      const int slot = L >> 3, per_row = groups * splits;
-      const int bb = (L & 7) + 8 * (slot / per_row), rem = slot % per_row;
-      unit = bb * groups + rem / splits;
-      split = rem % splits;
-    } else {
-      unit = L / splits;
-      split = L % splits;
-    }
-  }
-  const int b = unit / groups;
-  const int grp = unit % groups;
+  // Batch rows vary fastest, so that with the workgroups dealt to the 8 XCDs in
+  // turn a batch row's groups share XCDs (their L2) where 8 divides B or B
+  // divides 8, and the last groups come first: under the causal mask theirs are
+  // the longest ranges, and the short ones fill in at the end.
+  const int b = (int)blockIdx.x % B;
+  const int place = (int)blockIdx.x / B;
+  const int grp = groups - 1 - place / splits, split = place % splits;
+  const int unit = b * groups + grp;
   const int R = T * H;
   const int r_base = grp * kRows;
   const QueryPos pos_b = query_pos(positions, tree_base, b, T);
@@ -1889,14 +1879,9 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
   const long long quantum = p.kind == kKeySplit ? 32 * kKeyWaves : 64 * kKeySets;
   int splits = requested;
   if (splits <= 0) {
-    const long long cus = compute_units();
     const long long wgs = (long long)B * p.groups;
-    // One workgroup per compute unit.
-    long long s = (cus + wgs - 1) / wgs;
     const long long max_s = (span + quantum - 1) / quantum;
-    if (s > max_s) s = max_s;
-    if (s < 1) s = 1;
-    splits = (int)s;
+    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s < 4096 ? max_s : 4096, c == 64 && p.mbw == 1);
   }
   if (splits > 4096) return fail(WPTV_E_INVALID, "verify_attention: splits %d above 4096", splits);
   p.splits = splits;
@@ -1938,10 +1923,10 @@ template <int MB, bool TREE>
 void launch_m32(dim3 grid, hipStream_t stream, const unsigned short* q, const unsigned short* k, int64_t ksb,
                 int64_t ksn, const unsigned short* v, int64_t vsb, int64_t vsn, const int64_t* positions, int window,
                 const int64_t* tree_base, const uint64_t* ancestors, const float* sink, int T, int H, int N,
-                float scale_log2, int groups, int splits, int range_from_positions, int xcd_map, RowMap rows,
-                OutGate gate, unsigned short* out, int out_fm, float* lse, unsigned short* part_o, float* part_lse) {
+                float scale_log2, int B, int groups, int splits, int range_from_positions, RowMap rows, OutGate gate,
+                unsigned short* out, int out_fm, float* lse, unsigned short* part_o, float* part_lse) {
   hipLaunchKernelGGL((verify_attention_m32<128, MB, TREE>), grid, dim3(kKeySets * MB * 64), 0, stream, positions,
-                     tree_base, xcd_map, groups, splits, T, H, N, window, range_from_positions, k, ksb, ksn, v, vsb,
+                     tree_base, B, groups, splits, T, H, N, window, range_from_positions, k, ksb, ksn, v, vsb,
                      vsn, q, ancestors, sink, scale_log2, rows, gate, out, out_fm, lse, part_o, part_lse);
 }
 
@@ -2078,14 +2063,12 @@ int attend(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
     st = launched("verify_attention_keys");
   } else if (p.kind == kRowBlocks32) {
     const int from_positions = (window > 0 || p.groups > 1 || (flags & WPTV_ATTN_RANGE_FROM_POSITIONS)) ? 1 : 0;
-    // the kernel's XCD numbering puts batch row b on XCD b mod 8: a batch count that 8 divides
-    const int xcd_rows = B % 8 == 0 ? 1 : 0;
     auto* po = static_cast<unsigned short*>(part_o);
 #define WPTV_LAUNCH(MM)                                                                                         \
   (tree_base ? launch_m32<MM, true> : launch_m32<MM, false>)(                                                   \
       grid, stream, qb, kb, k_stride_b, k_stride_n, vb, v_stride_b, v_stride_n, positions, window, tree_base,   \
-      tree_ancestors, sink, T, H, N, scale_log2, p.groups, p.splits, from_positions, xcd_rows, rows, gate, ob,      \
-      out_fm, lse, po, part_lse)
+      tree_ancestors, sink, T, H, N, scale_log2, B, p.groups, p.splits, from_positions, rows, gate, ob, out_fm, \
+      lse, po, part_lse)
     switch (p.mbw / 2) {
       case 1: WPTV_LAUNCH(1); break;
       case 2: WPTV_LAUNCH(2); break;

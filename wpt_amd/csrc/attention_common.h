@@ -1,9 +1,10 @@
 // What the attention kernels share: the rows a query sees, where a logical row
-// sits in the table, and the output gate.
+// sits in the table, the output gate, and the parts a key range is split into.
 #pragma once
 
 #include "wptv_common.h"
 
+#include <algorithm>
 #include <climits>
 
 namespace wptv {
@@ -107,6 +108,38 @@ __device__ __forceinline__ float gate_factor(unsigned short g) {
 // o rounded to bf16, times the gate factor, rounded again.
 __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) {
   return f32_to_bf16(bf16_to_f32(f32_to_bf16(o)) * gate_factor(g));
+}
+
+// Key-range parts of each of `units` workgroups' `tiles` 32-row tiles (at most
+// max_splits).  A compute unit holds one workgroup of these kernels, so the
+// parts run in rounds of one a compute unit, and a last round of a few parts
+// costs as much as a whole one: the counts tried are those that fill one, two or
+// three rounds, and no split at all.  A round costs its parts' tiles and about
+// 12 tiles' time to start and merge, the combine launch about 7: measured, us,
+// the count before (a part more than fills one round) -> the rule's: batch 47 x
+// 1536 rows, 5 queries of 16 heads, 24.9 at 6 -> 16.4 at 5 (8 and 10: 23.8,
+// 24.5); 39 x 4500, 37.8 at 7 -> 24.4 at 6; 23 x 2031, 26.3 at 12 -> 17.4 at 11;
+// 48 x 5000, one query, 46.7 at 6 -> 29.6 at 5; prompts of 3 x 546 tokens, 31.6
+// at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.  Up to ten tiles one part
+// is as fast (batch 32 x 300: 12.6 at 3, 12.3 at 1; a window of 128: 11.7 at 2,
+// 10.1 at 1) and its one launch is 4 us less of a program that launches call by
+// call.  shared: a compute unit holds several workgroups of the form (head width
+// 64, one 16-row block) and a part over matters less (39 x 4500: 16.4 us at 7 parts,
+// 17.0 at 6).
+inline long long pick_splits(long long units, long long tiles, long long max_splits, bool shared = false) {
+  const long long cus = compute_units();
+  if (shared && units < cus && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
+  long long best = 1, best_cost = (tiles + 12) * ((units + cus - 1) / cus);
+  for (int rounds = 1; rounds <= 3; ++rounds) {
+    const long long s = std::min(rounds * cus / units, max_splits);
+    if (s <= 1) continue;
+    const long long cost = ((tiles + s - 1) / s + 12) * ((units * s + cus - 1) / cus) + 7;
+    if (cost < best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 }  // namespace
