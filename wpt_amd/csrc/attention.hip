@@ -2269,9 +2269,11 @@ int sparse_plan(int B, int T, int H, int c, int K, int window, int N, int dtype,
   const long long total = (long long)K + (window < N ? window : N);  // the longest list of a query
   long long s = requested;
   if (s <= 0) {
-    s = (compute_units() + (long long)B * T - 1) / ((long long)B * T);  // a workgroup per compute unit
-    const long long most = (total + 127) / 128;  // at least one tile per wavefront
-    if (s > most) s = most;
+    // Whole rounds of the compute units (pick_splits; a split's list is read 128 rows at a time, at least
+    // one tile a wavefront), us at 1024 chosen and 128 window rows, a part more than fills a round -> now:
+    // 160 queries 31.0 at 2 -> 24.0 at 1 (3 splits in two rounds 24.9), 100 25.3 at 3 -> 19.8 at 2, 50 18.3
+    // at 6 -> 13.5 at 5, 36 17.1 at 8 -> 12.1 at 7.
+    s = pick_splits((long long)B * T, (total + 31) / 32, (total + 127) / 128);
   }
   const long long least = (total + kSparseList - 1) / kSparseList;  // the list of a split fits its LDS
   if (s < least) s = least;

@@ -115,15 +115,15 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 // parts run in rounds of one a compute unit, and a last round of a few parts
 // costs as much as a whole one: the counts tried are those that fill one, two or
 // three rounds, and no split at all.  A round costs its parts' tiles and about
-// 12 tiles' time to start and merge, the combine launch about 7: measured, us,
+// 12 tiles' time to start and merge, the combine launch about 6: measured, us,
 // the count before (a part more than fills one round) -> the rule's: batch 47 x
 // 1536 rows, 5 queries of 16 heads, 24.9 at 6 -> 16.4 at 5 (8 and 10: 23.8,
 // 24.5); 39 x 4500, 37.8 at 7 -> 24.4 at 6; 23 x 2031, 26.3 at 12 -> 17.4 at 11;
 // 48 x 5000, one query, 46.7 at 6 -> 29.6 at 5; prompts of 3 x 546 tokens, 31.6
 // at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.  Up to ten tiles one part
-// is as fast (batch 32 x 300: 12.6 at 3, 12.3 at 1; a window of 128: 11.7 at 2,
-// 10.1 at 1) and its one launch is 4 us less of a program that launches call by
-// call.  shared: a compute unit holds several workgroups of the form (head width
+// is about as fast in a graph (batch 32 x 300: 12.6 at 3, 12.3 at 1; batch 1: 11.3,
+// 11.8; a window of 128: 11.7 at 2, 10.1 at 1) and its one launch is 4 us less of a
+// program that launches call by call (batch 1 x 300: 16.8 -> 12.6).  shared: a compute unit holds several workgroups of the form (head width
 // 64, one 16-row block) and a part over matters less (39 x 4500: 16.4 us at 7 parts,
 // 17.0 at 6).
 inline long long pick_splits(long long units, long long tiles, long long max_splits, bool shared = false) {
@@ -133,7 +133,7 @@ inline long long pick_splits(long long units, long long tiles, long long max_spl
   for (int rounds = 1; rounds <= 3; ++rounds) {
     const long long s = std::min(rounds * cus / units, max_splits);
     if (s <= 1) continue;
-    const long long cost = ((tiles + s - 1) / s + 12) * ((units * s + cus - 1) / cus) + 7;
+    const long long cost = ((tiles + s - 1) / s + 12) * ((units * s + cus - 1) / cus) + 6;
     if (cost < best_cost) {
       best = s;
       best_cost = cost;

@@ -383,15 +383,16 @@ void launch_width(const F32Plan& p, const F32Call& a, float* part_o, float* part
 
 bool attention_f32_takes(int c) { return c == 64 || c == 128; }
 
-// One workgroup per compute unit where the keys allow it, each wavefront at
-// least one tile.  Measured on the MI355X, graph replays, us a call (batch,
-// queries, heads, width, rows): the wave-per-query kernel, then this one
-//   (8, 5, 4, 64, 1029)     366   10.2
-//   (1, 5, 4, 64, 300)      103    8.0
-//   (8, 9, 16, 128, 2048)  1937    33
-//   (2, 200, 8, 64, 700)    369    17
-//   (1, 5, 16, 128, 2048)  1129    13.6
-//   (2, 33, 4, 64, 33)       16    5.2
+// Whole rounds of one workgroup per compute unit (pick_splits), each wavefront
+// at least one tile.  Measured on the MI355X, graph replays, us a call (batch,
+// queries, heads, width, rows): the wave-per-query kernel, this one with a
+// part more than fills the round, this one
+//   (8, 5, 4, 64, 1029)     366   10.2  10.2
+//   (1, 5, 4, 64, 300)      103    7.7   7.7
+//   (4, 6, 16, 128, 1769)         20.4  15.5
+//   (8, 9, 16, 128, 2048)  1937   32.3  26.8
+//   (2, 200, 8, 64, 700)    369   18.1  15.4
+//   (2, 175, 4, 64, 175)           8.6   7.4
 // A wavefront holding two to five row blocks (each key read by fewer
 // workgroups) was slower at all of these: 12.4-50 us, one wavefront a SIMD.
 F32Plan attention_f32_plan(int B, int T, int H, int c, int N, int window, int requested) {
@@ -401,7 +402,7 @@ F32Plan attention_f32_plan(int B, int T, int H, int c, int N, int window, int re
   if (window > 0 && (long long)window + T - 1 < span) span = (long long)window + T - 1;
   const long long max_splits = (span + kF32Tile * kF32Waves - 1) / (kF32Tile * kF32Waves);
   const long long units = (long long)B * p.groups;
-  long long s = requested > 0 ? requested : (compute_units() + units - 1) / units;
+  long long s = requested > 0 ? requested : pick_splits(units, (span + 31) / 32, max_splits);
   if (s > max_splits) s = max_splits;
   if (s < 1) s = 1;
   p.splits = (int)s;
