@@ -199,7 +199,14 @@ __device__ __forceinline__ float group_sum(float x) {
 // the first key range depends on come first: gfx950 preloads a kernel's first
 // 14 argument dwords into SGPRs, so the positions load is issued at once and
 // the rest of the arguments arrive meanwhile.
-template <int C, int MB, bool TREE>
+//
+// ROWS: the query rows of a group (and of its parts).  At head width 128 up to
+// 16 rows (one query of 16 heads) run with a second wavefront a key set whose
+// block is padding: one wavefront alone issues a key set's DMA too slowly
+// (ROWS = 16 < 16 MB; one group only).  Batch 48 x 5000 rows, 36.2 in the place
+// of 42.9 us at the same parts, 32 x 4100 15.3 and 16.7; at head width 64, half
+// the DMA, 13.7 and 12.9.
+template <int C, int MB, bool TREE, int ROWS = 16 * MB>
 __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
     const int64_t* __restrict__ positions, const int64_t* __restrict__ tree_base, int xcd_map, int groups,
     int splits, int T, int H, int N, int window, int range_from_positions, const unsigned short* __restrict__ k,
@@ -208,7 +215,7 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
     float scale_log2, RowMap rows, OutGate gate, unsigned short* __restrict__ out, int out_fm,
     float* __restrict__ lse_out, unsigned short* __restrict__ part_o, float* __restrict__ part_lse) {
   using G = Tile<C>;
-  constexpr int kRows = 16 * MB;
+  constexpr int kRows = ROWS;
   constexpr int kXC = C / 8;  // 16-byte chunks per key or value row
   constexpr int DMAW = MB >= 4 ? 4 : (MB >= 2 ? 2 : 1);  // wavefronts of a key set that issue its DMA
   constexpr int kCnt = G::kLoads / DMAW;                 // DMA instructions per such wavefront and tile
@@ -1907,14 +1914,14 @@ void launch_keys(dim3 grid, hipStream_t stream, const unsigned short* q, const u
                      xcd_map, out, lse, part_o, part_lse);
 }
 
-template <int C, int MBW, bool TREE>
+template <int C, int MBW, bool TREE, int ROWS>
 void launch_mfma(dim3 grid, hipStream_t stream, const unsigned short* q, const unsigned short* k, int64_t ksb,
                  int64_t ksn, const unsigned short* v, int64_t vsb, int64_t vsn, const int64_t* positions,
                  int window, const int64_t* tree_base, const uint64_t* ancestors, const float* sink, int T, int H,
                  int N, float scale_log2, int groups, int splits, int range_from_positions, int xcd_map,
                  RowMap rows, OutGate gate, unsigned short* out, int out_fm, float* lse, unsigned short* part_o,
                  float* part_lse) {
-  hipLaunchKernelGGL((verify_attention_mfma<C, MBW, TREE>), grid, dim3(kKeySets * MBW * 64), 0, stream, positions,
+  hipLaunchKernelGGL((verify_attention_mfma<C, MBW, TREE, ROWS>), grid, dim3(kKeySets * MBW * 64), 0, stream, positions,
                      tree_base, xcd_map, groups, splits, T, H, N, window, range_from_positions, k, ksb, ksn, v, vsb,
                      vsn, q, ancestors, sink, scale_log2, rows, gate, out, out_fm, lse, part_o, part_lse);
 }
@@ -2084,14 +2091,15 @@ int attend(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
     // the kernel's XCD numbering puts batch row b on XCD b mod 8: a batch count that 8 divides
     const int xcd_rows = B % 8 == 0 ? 1 : 0;
     auto* po = static_cast<unsigned short*>(part_o);
-#define WPTV_LAUNCH(CC, MM)                                                                                     \
-  (tree_base ? launch_mfma<CC, MM, true> : launch_mfma<CC, MM, false>)(                                         \
+#define WPTV_FORM(CC, MM, ROWS)                                                                                 \
+  (tree_base ? launch_mfma<CC, MM, true, ROWS> : launch_mfma<CC, MM, false, ROWS>)(                             \
       grid, stream, qb, kb, k_stride_b, k_stride_n, vb, v_stride_b, v_stride_n, positions, window, tree_base,   \
       tree_ancestors, sink, T, H, N, scale_log2, p.groups, p.splits, from_positions, xcd_rows, rows, gate, ob,      \
       out_fm, lse, po, part_lse)
+#define WPTV_LAUNCH(CC, MM) WPTV_FORM(CC, MM, 16 * MM)
     if (c == 128) {
       switch (p.mbw) {
-        case 1: WPTV_LAUNCH(128, 1); break;
+        case 1: WPTV_FORM(128, 2, 16); break;
         case 2: WPTV_LAUNCH(128, 2); break;
         case 3: WPTV_LAUNCH(128, 3); break;
         case 4: WPTV_LAUNCH(128, 4); break;
@@ -2109,6 +2117,7 @@ int attend(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
       }
     }
 #undef WPTV_LAUNCH
+#undef WPTV_FORM
     st = launched("verify_attention_mfma");
   }
   if (st != WPTV_OK || p.splits == 1) return st;
