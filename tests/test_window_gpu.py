@@ -204,3 +204,47 @@ def test_a_reading_wider_than_the_rings_must_not_be_undoable(device):
     cache = gpu.new_cache(1, widest=8)
     with pytest.raises(ValueError):
         gpu.extend(torch.zeros(1, 40, dtype=torch.long, device=device), cache, undoable=True)
+
+
+@pytest.mark.parametrize("T, H, c", [(1, 16, 128), (3, 11, 128), (8, 16, 128), (9, 16, 128), (31, 16, 128), (5, 7, 64),
+                                     (17, 8, 64)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_every_row_block_form_gates_its_output(device, T, H, c, splits):
+    # one part gates in the attention kernel (each row-block form, padding rows in its last block), two
+    # in the merge: o rounded to bf16, times sigmoid(gate) rounded to bf16, rounded again, so within
+    # 3 bf16 half steps of the FP32 formula but for the probabilities' own rounding
+    B, window, start = 2, 128, 300
+    q = draw(B, T, H, c, seed=31)
+    full = draw(B, start + T, 2 * c, seed=32)
+    sink = draw(H, seed=33, dtype=torch.float32)
+    proj = draw(B, T, (2 * H + 2) * c, seed=34)
+    gate = proj[..., (H + 2) * c:]
+    positions = (start + torch.arange(T)).expand(B, T)
+    ring = torch.zeros(B, 256, 2 * c, dtype=torch.bfloat16)
+    held = torch.arange(start + T - 256, start + T)
+    ring[:, held % 256] = full[:, held]
+    table = tail_table(full, start, window)
+    expected = oracle.window_attention(q, table[..., :c], table[..., c:], sink, positions, c ** -0.5, window)
+    expected = expected * torch.sigmoid(gate.float()).reshape(B, T, H, c)
+    got = kernels.ring_attention(q.to(device), ring.to(device), positions.to(device), c ** -0.5, window,
+                                 sink.to(device), gate=proj.to(device)[..., (H + 2) * c:], splits=splits)
+    assert relative_error(got.cpu(), expected) < 2e-2
+
+
+def test_every_bf16_gate(device):
+    # one visible value of 1 a query: the output is the gate's factor itself, sigmoid(gate) rounded to
+    # bf16 (half a step, 2^-9 of it, and the FP32 exponential's own error); where exp(-gate) passes FP32's
+    # largest value, 2^128, it is infinite and the factor 0: factors below 2^-128
+    H, c = 16, 128
+    gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).reshape(-1, 1, H * c)
+    B = gate.shape[0]
+    ring = torch.zeros(B, 256, 2 * c, dtype=torch.bfloat16)
+    ring[..., c:] = 1.0
+    q = torch.zeros(B, 1, H, c, dtype=torch.bfloat16)
+    got = kernels.ring_attention(q.to(device), ring.to(device), torch.zeros(B, 1, dtype=torch.long, device=device),
+                                 c ** -0.5, 128, torch.full((H,), -1e30, device=device), gate=gate.to(device))
+    want = torch.sigmoid(gate.double()).flatten()
+    got = got.cpu().double().flatten()
+    assert torch.equal(got.isnan(), want.isnan())
+    known = ~want.isnan()
+    assert ((got - want).abs()[known] <= 2.0 ** -8 * want[known] + 2.0 ** -128).all()

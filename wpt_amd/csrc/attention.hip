@@ -539,14 +539,19 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
     const unsigned short* grow = gate.row<unsigned short>(b, T, r, H, C);
     // out_fm > 0: the output [B T, H C] in the fm layout with out_fm row blocks
     const int fm_row = b * T + r / H, fm_col = (r % H) * C;
+    // every gate value before the first store: where it is used, each load waited for the store before it
+    u16x4 gv[G::kCBlocks];
+    if (grow) {
+#pragma unroll
+      for (int cb = 0; cb < G::kCBlocks; ++cb) gv[cb] = *reinterpret_cast<const u16x4*>(grow + cb * 16 + 4 * g);
+    }
 #pragma unroll
     for (int cb = 0; cb < G::kCBlocks; ++cb) {
       const f32x4 val = o[cb] * scale_out;
       u16x4 res;
       if (grow) {
-        const u16x4 gv = *reinterpret_cast<const u16x4*>(grow + cb * 16 + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) res[e] = gated_bf16(val[e], gv[e]);
+        for (int e = 0; e < 4; ++e) res[e] = gated_bf16(val[e], gv[cb][e]);
       } else {
         res = u16x4{f32_to_bf16(val[0]), f32_to_bf16(val[1]), f32_to_bf16(val[2]), f32_to_bf16(val[3])};
       }
@@ -918,6 +923,12 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
     unsigned short* orow = out + ((int64_t)b * R + r) * C;
     const unsigned short* grow = gate.row<unsigned short>(b, T, r, H, C);
     const int fm_row = b * T + r / H, fm_col = (r % H) * C;
+    // every gate value before the first store, as verify_attention_mfma (31 queries, 21.4 -> 20.0 us)
+    u16x4 gv[4 * kCB];
+    if (grow) {
+#pragma unroll
+      for (int i = 0; i < 4 * kCB; ++i) gv[i] = *reinterpret_cast<const u16x4*>(grow + 8 * i + 4 * h);
+    }
 #pragma unroll
     for (int cb = 0; cb < kCB; ++cb)
 #pragma unroll
@@ -925,9 +936,8 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
         const int c0 = 32 * cb + 8 * a + 4 * h;
         u16x4 res;
         if (grow) {
-          const u16x4 gv = *reinterpret_cast<const u16x4*>(grow + c0);
 #pragma unroll
-          for (int m = 0; m < 4; ++m) res[m] = gated_bf16(o[cb][4 * a + m] * scale_out, gv[m]);
+          for (int m = 0; m < 4; ++m) res[m] = gated_bf16(o[cb][4 * a + m] * scale_out, gv[4 * cb + a][m]);
         } else {
 #pragma unroll
           for (int m = 0; m < 4; ++m) res[m] = f32_to_bf16(o[cb][4 * a + m] * scale_out);

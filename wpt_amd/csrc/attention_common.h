@@ -101,13 +101,22 @@ struct OutGate {
   }
 };
 
+// Few instructions, since a call of one part has few wavefronts to gate with (a
+// lane of the 32-row blocks gates 64 columns): with a division and the rounding
+// in integers a window of 128 took, graph replays, us, in one part and in the two
+// parts that this replaced, then in one part as here: batch 32, 5 queries of 16
+// heads 15.7, 13.3, 11.5; batch 16, 31 queries 21.4, 16.1, 13.2.  The reciprocal is
+// v_rcp_f32 of a quarter of the denominator, a quarter of that again, so that a
+// subnormal factor is kept; each of the 65536 gates gives the division's bits.
+__device__ __forceinline__ float round_bf16(float f) { return static_cast<float>(static_cast<__bf16>(f)); }
+
 __device__ __forceinline__ float gate_factor(unsigned short g) {
-  return bf16_to_f32(f32_to_bf16(1.f / (1.f + __expf(-bf16_to_f32(g)))));
+  return round_bf16(0.25f * __builtin_amdgcn_rcpf(0.25f + 0.25f * __expf(-bf16_to_f32(g))));
 }
 
 // o rounded to bf16, times the gate factor, rounded again.
 __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) {
-  return f32_to_bf16(bf16_to_f32(f32_to_bf16(o)) * gate_factor(g));
+  return __builtin_bit_cast(unsigned short, static_cast<__bf16>(round_bf16(o) * gate_factor(g)));
 }
 
 // Key-range parts of each of `units` workgroups' `tiles` 32-row tiles (at most
