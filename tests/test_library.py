@@ -55,3 +55,25 @@ def test_bad_arguments_are_reported_with_a_message():
     status = library.wptv_attention_workspace(1, 1, 1, 128, 8, 0, 7, 0, ctypes.byref(splits), ctypes.byref(size))
     with pytest.raises(NotImplementedError):
         _lib.check(status, "attention_workspace")
+
+
+def chosen_parts(B, T, H, c, N, window=0, dtype=_lib.WPTV_BF16, flags=_lib.RANGE_FROM_POSITIONS):
+    splits, size = ctypes.c_int(0), ctypes.c_size_t(0)
+    assert _lib.lib().wptv_attention_workspace(B, T, H, c, N, window, dtype, flags, ctypes.byref(splits),
+                                               ctypes.byref(size)) == 0
+    return splits.value
+
+
+@pytest.mark.parametrize("B, T, N", [(256, 5, 4100), (257, 5, 4100), (300, 5, 4100), (384, 5, 8000), (4, 600, 3600),
+                                     (300, 1, 5000)])
+def test_a_call_that_fills_the_compute_units_has_one_bf16_rounding(B, T, N):
+    # parts are held in bf16: where a workgroup a (batch row, query group) fills the 256 compute units, a
+    # second part would only add its rounding (the sums of one part are FP32 throughout)
+    assert chosen_parts(B, T, 16, 128, N) == 1
+
+
+def test_sparse_calls_that_fill_the_compute_units_have_one_bf16_rounding():
+    splits, size = ctypes.c_int(0), ctypes.c_size_t(0)
+    assert _lib.lib().wptv_sparse_attention_workspace(60, 5, 16, 128, 3900, 128, 20000, _lib.WPTV_BF16,
+                                                      ctypes.byref(splits), ctypes.byref(size)) == 0
+    assert splits.value == 1

@@ -1898,7 +1898,7 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
   if (splits <= 0) {
     const long long wgs = (long long)B * p.groups;
     const long long max_s = (span + quantum - 1) / quantum;
-    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s < 4096 ? max_s : 4096, c == 64 && p.mbw == 1);
+    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s < 4096 ? max_s : 4096, false, c == 64 && p.mbw == 1);
   }
   if (splits > 4096) return fail(WPTV_E_INVALID, "verify_attention: splits %d above 4096", splits);
   p.splits = splits;
@@ -2292,7 +2292,7 @@ int sparse_plan(int B, int T, int H, int c, int K, int window, int N, int dtype,
     // one tile a wavefront), us at 1024 chosen and 128 window rows, a part more than fills a round -> now:
     // 160 queries 31.0 at 2 -> 24.0 at 1 (3 splits in two rounds 24.9), 100 25.3 at 3 -> 19.8 at 2, 50 18.3
     // at 6 -> 13.5 at 5, 36 17.1 at 8 -> 12.1 at 7.
-    s = pick_splits((long long)B * T, (total + 31) / 32, (total + 127) / 128);
+    s = pick_splits((long long)B * T, (total + 31) / 32, (total + 127) / 128, false);
   }
   const long long least = (total + kSparseList - 1) / kSparseList;  // the list of a split fits its LDS
   if (s < least) s = least;

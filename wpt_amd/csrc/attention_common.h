@@ -120,8 +120,8 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 }
 
 // Key-range parts of each of `units` workgroups' `tiles` 32-row tiles (at most
-// max_splits).  A compute unit holds one workgroup of these kernels, so the
-// parts run in rounds of one a compute unit, and a last round of a few parts
+// max_splits).  A compute unit holds one workgroup of most of these kernels, so
+// the parts run in rounds of one a compute unit, and a last round of a few parts
 // costs as much as a whole one: the counts tried are those that fill one, two or
 // three rounds, and no split at all.  A round costs its parts' tiles and about
 // 12 tiles' time to start and merge, the combine launch about 6: measured, us,
@@ -129,15 +129,25 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 // 1536 rows, 5 queries of 16 heads, 24.9 at 6 -> 16.4 at 5 (8 and 10: 23.8,
 // 24.5); 39 x 4500, 37.8 at 7 -> 24.4 at 6; 23 x 2031, 26.3 at 12 -> 17.4 at 11;
 // 48 x 5000, one query, 46.7 at 6 -> 29.6 at 5; prompts of 3 x 546 tokens, 31.6
-// at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.  Up to ten tiles one part
-// is about as fast in a graph (batch 32 x 300: 12.6 at 3, 12.3 at 1; batch 1: 11.3,
-// 11.8; a window of 128: 11.7 at 2, 10.1 at 1) and its one launch is 4 us less of a
-// program that launches call by call (batch 1 x 300: 16.8 -> 12.6).  shared: a compute unit holds several workgroups of the form (head width
-// 64, one 16-row block) and a part over matters less (39 x 4500: 16.4 us at 7 parts,
+// at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.  Up to ten tiles one
+// part is about as fast in a graph (batch 32 x 300: 12.6 at 3, 12.3 at 1; batch
+// 1: 11.3, 11.8) and its one launch is 4 us less of a program that launches call
+// by call (batch 1 x 300: 16.8 -> 12.6).
+//
+// fp32_parts: the parts are held in FP32.  Parts of bf16 add a rounding each, so
+// where one part a unit fills the compute units the range stays whole, although
+// two were faster (batch 257 x 4100, 5 queries of 16 heads: 150 us, 131 in two,
+// 300: 153, 134; 4 prompts of 600 tokens over 3600 rows 125, 116): outputs over
+// 3600 rows are off by 0.00235 of their norm in one part, 0.0029 in two.
+//
+// shared: a compute unit holds several workgroups of the form (head width 64,
+// one 16-row block) and a part over matters less (39 x 4500: 16.4 us at 7 parts,
 // 17.0 at 6).
-inline long long pick_splits(long long units, long long tiles, long long max_splits, bool shared = false) {
+inline long long pick_splits(long long units, long long tiles, long long max_splits, bool fp32_parts,
+                             bool shared = false) {
   const long long cus = compute_units();
-  if (shared && units < cus && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
+  if (!fp32_parts && units >= cus) return 1;
+  if (shared && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
   long long best = 1, best_cost = (tiles + 12) * ((units + cus - 1) / cus);
   for (int rounds = 1; rounds <= 3; ++rounds) {
     const long long s = std::min(rounds * cus / units, max_splits);

@@ -402,7 +402,7 @@ F32Plan attention_f32_plan(int B, int T, int H, int c, int N, int window, int re
   if (window > 0 && (long long)window + T - 1 < span) span = (long long)window + T - 1;
   const long long max_splits = (span + kF32Tile * kF32Waves - 1) / (kF32Tile * kF32Waves);
   const long long units = (long long)B * p.groups;
-  long long s = requested > 0 ? requested : pick_splits(units, (span + 31) / 32, max_splits);
+  long long s = requested > 0 ? requested : pick_splits(units, (span + 31) / 32, max_splits, true);
   if (s > max_splits) s = max_splits;
   if (s < 1) s = 1;
   p.splits = (int)s;
