@@ -113,11 +113,12 @@ int wptv_verify_attention(const void* q, const void* k, int64_t k_stride_b, int6
  *   graph capture, tight serving loops, harnesses that forbid hipMalloc).  It
  *   has no counterpart in the reference.  The key-range parts live in a
  *   static device array of 16 MiB that each device loading the library holds
- *   until the process ends (enough for every split count the library
- *   chooses for c <= 128; a request needing more is refused with
- *   WPTV_E_INVALID and a message).  It calls no allocating routine.  Calls
- *   that overlap on one device share that array and race; calls ordered on
- *   one stream do not.  Same kernels and results as wptv_verify_attention. */
+ *   until the process ends: splits 0 takes the best count whose parts fit it,
+ *   a count whose parts do not is refused with WPTV_E_INVALID and a message.
+ *   FP32 calls run in one part.  It calls no allocating routine.  Calls that
+ *   overlap on one device share that array and race; calls ordered on one
+ *   stream do not.  Same kernels as wptv_verify_attention, and the same results
+ *   at the same count. */
 int wptv_verify_attention_static(const void* q, const void* k, int64_t k_stride_b, int64_t k_stride_n,
                                  const void* v, int64_t v_stride_b, int64_t v_stride_n, int dtype,
                                  const int64_t* positions, int window, const int64_t* tree_base,

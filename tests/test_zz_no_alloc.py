@@ -59,10 +59,9 @@ def test_a_request_beyond_the_static_scratch_is_refused(device):
 
 
 def test_the_library_s_own_split_count_steps_down_to_fit(device):
-    # 255 batch rows of 128 query rows: the library's choice for the workspace
-    # entry point is 2 splits, whose parts (17 MB) do not fit the static array;
-    # the allocation-free entry point takes one split instead, the same bits as
-    # the workspace entry point asked for one split
+    # 255 batch rows of 128 query rows: two splits, whose parts (17 MB) do not
+    # fit the static array, are not chosen; the same bits as the workspace entry
+    # point asked for one split
     B, T, H, c, N = 255, 8, 16, 128, 300
     print(f"static scratch step-down: B={B} T={T} H={H} c={c} N={N}", flush=True)
     q, table, positions = (x.to(device) for x in inputs(B, T, H, c, N, seed=11))
@@ -71,3 +70,17 @@ def test_the_library_s_own_split_count_steps_down_to_fit(device):
     expected = kernels.verify_attention(q, k, v, positions, c ** -0.5, splits=1)
     torch.cuda.synchronize()
     assert torch.equal(got, expected)
+
+
+def test_the_library_s_own_split_count_is_the_best_that_fits(device):
+    # 171 units of 128 query rows: the workspace entry point's choice, four splits in three rounds of
+    # the compute units, takes 21.7 MiB.  Two fit, but run in two rounds: of the counts that fit, one is
+    # the choice.  The same bits as the workspace entry point asked for one split
+    B, T, H, c, N = 19, 72, 16, 128, 4200
+    print(f"static scratch choice: B={B} T={T} H={H} c={c} N={N}", flush=True)
+    q, table, positions = (x.to(device) for x in inputs(B, T, H, c, N, seed=12))
+    k, v = table[..., :c], table[..., c:]
+    got = kernels.verify_attention(q, k, v, positions, c ** -0.5, static_scratch=True)
+    expected = [kernels.verify_attention(q, k, v, positions, c ** -0.5, splits=s) for s in (1, 2)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, expected[0]) and not torch.equal(*expected)

@@ -1833,7 +1833,9 @@ int pick_mbw(int R) {
   return 8;
 }
 
-int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, int requested, Plan* out) {
+// max_bytes: the parts of a count of the library's choosing fit in that many.
+int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, int requested, Plan* out,
+         size_t max_bytes = SIZE_MAX) {
   if (B <= 0 || T <= 0 || H <= 0 || c <= 0 || N <= 0)
     return fail(WPTV_E_INVALID, "verify_attention: B, T, H, c and N must be positive (got %d, %d, %d, %d, %d)", B,
                 T, H, c, N);
@@ -1897,8 +1899,10 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
   int splits = requested;
   if (splits <= 0) {
     const long long wgs = (long long)B * p.groups;
-    const long long max_s = (span + quantum - 1) / quantum;
-    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s < 4096 ? max_s : 4096, false, c == 64 && p.mbw == 1);
+    long long max_s = std::min((span + quantum - 1) / quantum, 4096LL);
+    const size_t part = (size_t)wgs * 16 * p.mbw * (c * 2 + sizeof(float));  // a part of every unit
+    if (max_bytes < (size_t)max_s * part + 512) max_s = max_bytes < 512 + part ? 1 : (long long)((max_bytes - 512) / part);
+    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s, false, c == 64 && p.mbw == 1);
   }
   if (splits > 4096) return fail(WPTV_E_INVALID, "verify_attention: splits %d above 4096", splits);
   p.splits = splits;
@@ -2205,17 +2209,12 @@ extern "C" int wptv_verify_attention_static(const void* q, const void* k, int64_
                                             const uint64_t* tree_ancestors, const float* sink, int B, int T, int H,
                                             int c, int N, float scale, int splits, int flags, void* out, float* lse,
                                             hipStream_t stream) {
+  // A count of the library's choosing is chosen among those whose parts fit the static array (one part needs none).
   Plan p;
-  int st = plan(B, T, H, c, N, window, dtype, flags, splits, &p);
+  int st = plan(B, T, H, c, N, window, dtype, flags, splits, &p, kScratchBytes);
   if (st == WPTV_OK && p.kind == kF32Mfma)  // FP32 calls keep no parts there, so that overlapping ones do not race
-    st = plan(B, T, H, c, N, window, dtype, flags, splits = 1, &p);
+    st = plan(B, T, H, c, N, window, dtype, flags, 1, &p);
   if (st != WPTV_OK) return st;
-  // a split count of the library's choosing steps down until its parts fit
-  // the static array (one split needs none)
-  while (splits <= 0 && p.bytes > kScratchBytes && p.splits > 1) {
-    st = plan(B, T, H, c, N, window, dtype, flags, p.splits - 1, &p);
-    if (st != WPTV_OK) return st;
-  }
   if (p.bytes > kScratchBytes)
     return fail(WPTV_E_INVALID,
                 "verify_attention_static: B=%d T=%d H=%d c=%d in %d splits needs %zu bytes of parts, above the %zu "
