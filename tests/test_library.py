@@ -77,3 +77,12 @@ def test_sparse_calls_that_fill_the_compute_units_have_one_bf16_rounding():
     assert _lib.lib().wptv_sparse_attention_workspace(60, 5, 16, 128, 3900, 128, 20000, _lib.WPTV_BF16,
                                                       ctypes.byref(splits), ctypes.byref(size)) == 0
     assert splits.value == 1
+
+
+@pytest.mark.parametrize("B, T, H, N, parts", [
+    (200, 2, 16, 4100, 2), (171, 2, 16, 2048, 2), (100, 2, 16, 3000, 5), (150, 4, 8, 1500, 3),  # two workgroups a unit
+    (200, 2, 16, 1029, 1), (23, 2, 16, 4100, 11), (255, 2, 16, 2048, 1),  # a part over costs more than it gives
+    (100, 3, 16, 4100, 5), (47, 5, 16, 4100, 5), (171, 3, 16, 1500, 1),   # three blocks and more: a round each
+    (39, 1, 16, 4500, 7)])                                               # one block: the parts cover the units
+def test_the_parts_at_head_width_64(B, T, H, N, parts):
+    assert chosen_parts(B, T, H, 64, N) == parts

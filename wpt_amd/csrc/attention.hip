@@ -1902,7 +1902,10 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
     long long max_s = std::min((span + quantum - 1) / quantum, 4096LL);
     const size_t part = (size_t)wgs * 16 * p.mbw * (c * 2 + sizeof(float));  // a part of every unit
     if (max_bytes < (size_t)max_s * part + 512) max_s = max_bytes < 512 + part ? 1 : (long long)((max_bytes - 512) / part);
-    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s, false, c == 64 && p.mbw == 1);
+    const Second second = c != 64 || p.kind != kRowBlocks || p.mbw > 2 ? Second::kRound
+                          : p.mbw == 2                               ? Second::kHalfRound
+                                                                     : Second::kFree;
+    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s, false, second);
   }
   if (splits > 4096) return fail(WPTV_E_INVALID, "verify_attention: splits %d above 4096", splits);
   p.splits = splits;

@@ -140,19 +140,36 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 // 300: 153, 134; 4 prompts of 600 tokens over 3600 rows 125, 116): outputs over
 // 3600 rows are off by 0.00235 of their norm in one part, 0.0029 in two.
 //
-// shared: a compute unit holds several workgroups of the form (head width 64,
-// one 16-row block) and a part over matters less (39 x 4500: 16.4 us at 7 parts,
-// 17.0 at 6).
+// Where a compute unit holds two workgroups of a form at once, a second one costs
+// less than a round (kHalfRound; the figures at head width 64, where each form
+// fits twice, are us at the counts in brackets).  One 16-row block: a part over
+// one a compute unit matters so little that the parts just cover the compute
+// units (39 x 4500 16.4 [7], 17.0 [6]).  Two blocks: a second workgroup adds 0.8
+// of a round, in proportion to how many compute units have one (200 x 4100 49.7
+// [1], 43.2 [2]; 100 x 3000 25.0 [2], 23.6 [3], 20.9 [5]; 150 x 1500 20.6 [1], 20.0
+// [2], 18.2 [3]; 23 x 4100 13.6 [11], 15.0 [22]).  Three blocks and more, and the
+// sparse form: their arithmetic fills a compute unit, and a second workgroup
+// costs a round (three blocks, 100 x 4100 33.2 [2], 41.9 [3]; 47 x 4100 19.2 [5],
+// 26.8 [6]; sparse, 160 queries 17.1 [1], 20.3 [2]).
+enum class Second { kRound, kHalfRound, kFree };
+
 inline long long pick_splits(long long units, long long tiles, long long max_splits, bool fp32_parts,
-                             bool shared = false) {
+                             Second second = Second::kRound) {
   const long long cus = compute_units();
   if (!fp32_parts && units >= cus) return 1;
-  if (shared && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
-  long long best = 1, best_cost = (tiles + 12) * ((units + cus - 1) / cus);
+  if (second == Second::kFree && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
+  auto rounds_of = [&](long long parts) {
+    if (second == Second::kRound) return (double)((parts + cus - 1) / cus);
+    const long long pairs = parts / (2 * cus), rest = parts % (2 * cus);
+    const double last = rest > cus ? 1.0 + 0.8 * (double)(rest - cus) / (double)cus : rest > 0 ? 1.0 : 0.0;
+    return 1.8 * (double)pairs + last;
+  };
+  long long best = 1;
+  double best_cost = (double)(tiles + 12) * rounds_of(units);
   for (int rounds = 1; rounds <= 3; ++rounds) {
     const long long s = std::min(rounds * cus / units, max_splits);
     if (s <= 1) continue;
-    const long long cost = ((tiles + s - 1) / s + 12) * ((units * s + cus - 1) / cus) + 6;
+    const double cost = (double)((tiles + s - 1) / s + 12) * rounds_of(units * s) + 6.0;
     if (cost < best_cost) {
       best = s;
       best_cost = cost;
