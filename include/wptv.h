@@ -57,9 +57,12 @@ enum {
   WPTV_ATTN_OUT_FM = 8,               /* the output as the output projection's operand: [B T, H c] in the
                                          fragment-major layout (below) with wptv_fm_row_blocks(B T) row blocks;
                                          bf16 row-block kernels only */
-  WPTV_ATTN_ROWS32 = 16               /* head width 128: the row-block kernel on 32-row blocks (each wavefront
+  WPTV_ATTN_ROWS32 = 16,              /* head width 128: the row-block kernel on 32-row blocks (each wavefront
                                          holds 32 query rows, v_mfma_f32_32x32x16_bf16), which is the default
                                          above 128 query rows (T*H) a batch row */
+  WPTV_ATTN_CALL_BY_CALL = 32         /* splits 0: the program launches call by call and the GPU waits for it, so
+                                         a short range runs in one part and one launch; by default the part
+                                         count is the GPU's own best, as in a captured graph */
 };
 
 int wptv_abi_version(void);

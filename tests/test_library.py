@@ -86,3 +86,13 @@ def test_sparse_calls_that_fill_the_compute_units_have_one_bf16_rounding():
     (39, 1, 16, 4500, 7)])                                               # one block: the parts cover the units
 def test_the_parts_at_head_width_64(B, T, H, N, parts):
     assert chosen_parts(B, T, H, 64, N) == parts
+
+
+@pytest.mark.parametrize("B, T, c, N, parts, alone", [
+    (1, 1, 128, 320, 3, 1), (64, 1, 128, 320, 3, 1), (128, 1, 128, 320, 1, 1), (1, 1, 128, 160, 1, 1),  # one block
+    (32, 2, 128, 288, 3, 1), (1, 5, 128, 300, 3, 1), (16, 5, 128, 320, 3, 1), (32, 5, 128, 320, 1, 1),
+    (1, 16, 128, 288, 3, 1), (8, 31, 128, 320, 1, 1), (1, 5, 64, 320, 1, 1),
+    (1, 5, 128, 700, 6, 6), (32, 5, 128, 4100, 8, 8)])
+def test_short_ranges_are_cut_for_graphs_and_left_whole_for_calls_one_by_one(B, T, c, N, parts, alone):
+    assert chosen_parts(B, T, 16, c, N) == parts
+    assert chosen_parts(B, T, 16, c, N, flags=_lib.RANGE_FROM_POSITIONS | _lib.CALL_BY_CALL) == alone

@@ -23,6 +23,7 @@ RANGE_FROM_POSITIONS = 2
 KEY_SPLIT = 4
 OUT_FM = 8
 ROWS32 = 16
+CALL_BY_CALL = 32
 
 
 class KernelUnavailable(RuntimeError):

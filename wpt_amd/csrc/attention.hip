@@ -1833,6 +1833,26 @@ int pick_mbw(int R) {
   return 8;
 }
 
+// The window entry points: a gated window in one part is the faster also in a
+// graph (batch 32, 5 queries of 16 heads 11.5 us, 12.6 in two).
+constexpr int kWindowFlags = WPTV_ATTN_RANGE_FROM_POSITIONS | WPTV_ATTN_CALL_BY_CALL;
+
+// What the combine launch costs the GPU itself, as pick_splits counts it, where
+// it decides: ranges of 7 to 10 tiles at head width 128, and batches that leave
+// it room beside them.  Measured in graphs, us in one part and in the two (256
+// rows) or three (288 rows and more) that fill the range: up to 16 query rows,
+// batch 1 x 320 10.4, 9.0, 64 x 320 11.2, 10.2, 128 x 320 11.7, 12.2; 17 to 48, 32 x
+// 320 10.7, 9.8; 49 to 128, 1 x 320 11.8, 11.2, 32 x 300 12.8, 13.0; 32-row blocks, 1
+// x 16 x 320 13.9, 12.4, 8 x 31 x 320 14.5, 14.7.  At head width 64 one part is the
+// faster throughout (5 queries of 16 heads, 32 x 320 10.0, 10.8).
+double graph_merge(int c, int R, long long units) {
+  if (c != 128 || units > 64) return 6.0;
+  if (R <= 16) return 2.0;
+  if (R <= 48) return 3.0;
+  if (units > 16) return 6.0;
+  return R <= 128 ? 5.0 : 3.0;
+}
+
 // max_bytes: the parts of a count of the library's choosing fit in that many.
 int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, int requested, Plan* out,
          size_t max_bytes = SIZE_MAX) {
@@ -1905,7 +1925,8 @@ int plan(int B, int T, int H, int c, int N, int window, int dtype, int flags, in
     const Second second = c != 64 || p.kind != kRowBlocks || p.mbw > 2 ? Second::kRound
                           : p.mbw == 2                               ? Second::kHalfRound
                                                                      : Second::kFree;
-    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s, false, second);
+    splits = (int)pick_splits(wgs, (span + 31) / 32, max_s, false,
+                              flags & WPTV_ATTN_CALL_BY_CALL || p.kind == kKeySplit ? 6.0 : graph_merge(c, R, wgs), second);
   }
   if (splits > 4096) return fail(WPTV_E_INVALID, "verify_attention: splits %d above 4096", splits);
   p.splits = splits;
@@ -2238,7 +2259,7 @@ extern "C" int wptv_window_attention_workspace(int B, int T, int H, int c, int w
   if (!splits || !bytes) return fail(WPTV_E_INVALID, "window_attention_workspace: null output pointer");
   if (window <= 0) return fail(WPTV_E_INVALID, "window_attention_workspace: window %d must be > 0", window);
   Plan p;
-  const int st = plan(B, T, H, c, window + T - 1, window, dtype, 0, *splits, &p);
+  const int st = plan(B, T, H, c, window + T - 1, window, dtype, kWindowFlags, *splits, &p);
   if (st != WPTV_OK) return st;
   *splits = p.splits;
   *bytes = p.bytes;
@@ -2263,7 +2284,7 @@ extern "C" int wptv_window_attention(const void* q, const void* k, int64_t k_str
   // Logical rows: token positions; the upper bound only keeps hi = p.
   const RowMap rows{row_base, row_base ? 0xffffffffu : (uint32_t)(ring_rows - 1)};
   return attend(q, k, k_stride_b, k_stride_n, v, v_stride_b, v_stride_n, dtype, positions, window, nullptr, nullptr,
-                sink, B, T, H, c, INT_MAX / 2, scale, splits, WPTV_ATTN_RANGE_FROM_POSITIONS, rows, ring_rows,
+                sink, B, T, H, c, INT_MAX / 2, scale, splits, kWindowFlags, rows, ring_rows,
                 OutGate{gate, gate_stride}, out, nullptr, workspace, workspace_bytes, stream);
 }
 
@@ -2317,7 +2338,7 @@ extern "C" int wptv_sparse_attention_workspace(int B, int T, int H, int c, int K
                                                int* splits, size_t* bytes) {
   if (!splits || !bytes) return fail(WPTV_E_INVALID, "sparse_attention_workspace: null output pointer");
   if (K == 0 && window > 0)  // the window alone: the row-block kernel (wptv_sparse_attention routes it there)
-    return wptv_attention_workspace(B, T, H, c, N, window, dtype, WPTV_ATTN_RANGE_FROM_POSITIONS, splits, bytes);
+    return wptv_attention_workspace(B, T, H, c, N, window, dtype, kWindowFlags, splits, bytes);
   SparsePlan p;
   const int st = sparse_plan(B, T, H, c, K, window, N, dtype, *splits, &p);
   if (st != WPTV_OK) return st;
@@ -2341,7 +2362,7 @@ extern "C" int wptv_sparse_attention(const void* q, const void* k, int64_t k_str
     return fail(WPTV_E_INVALID, "sparse_attention: gate row stride %lld below H*c", (long long)gate_stride);
   if (K == 0 && window > 0)  // no chosen rows: the window attention of the row-block kernel, reading the window only
     return attend(q, k, k_stride_b, k_stride_n, v, v_stride_b, v_stride_n, dtype, positions, window, nullptr, nullptr,
-                  sink, B, T, H, c, N, scale, splits, WPTV_ATTN_RANGE_FROM_POSITIONS, RowMap{nullptr, 0xffffffffu}, N,
+                  sink, B, T, H, c, N, scale, splits, kWindowFlags, RowMap{nullptr, 0xffffffffu}, N,
                   OutGate{gate, gate_stride}, out, lse, workspace, workspace_bytes, stream);
   SparsePlan p;
   int st = sparse_plan(B, T, H, c, K, window, N, dtype, splits, &p);

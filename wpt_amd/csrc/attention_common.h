@@ -124,15 +124,16 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 // the parts run in rounds of one a compute unit, and a last round of a few parts
 // costs as much as a whole one: the counts tried are those that fill one, two or
 // three rounds, and no split at all.  A round costs its parts' tiles and about
-// 12 tiles' time to start and merge, the combine launch about 6: measured, us,
+// 12 tiles' time to start and merge, the combine launch `merge` more: measured, us,
 // the count before (a part more than fills one round) -> the rule's: batch 47 x
 // 1536 rows, 5 queries of 16 heads, 24.9 at 6 -> 16.4 at 5 (8 and 10: 23.8,
 // 24.5); 39 x 4500, 37.8 at 7 -> 24.4 at 6; 23 x 2031, 26.3 at 12 -> 17.4 at 11;
 // 48 x 5000, one query, 46.7 at 6 -> 29.6 at 5; prompts of 3 x 546 tokens, 31.6
-// at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.  Up to ten tiles one
-// part is about as fast in a graph (batch 32 x 300: 12.6 at 3, 12.3 at 1; batch
-// 1: 11.3, 11.8) and its one launch is 4 us less of a program that launches call
-// by call (batch 1 x 300: 16.8 -> 12.6).
+// at 2 -> 21.1 at 1, of 1 x 925, 28.7 at 3 -> 23.1 at 2.
+//
+// merge: 6 where a program launches call by call (up to ten tiles then run in
+// one part: batch 1 x 300 17.5 us in three, 13.1 in one).  Less for the bf16
+// row-block kernels on the GPU alone, as in a graph (graph_merge).
 //
 // fp32_parts: the parts are held in FP32.  Parts of bf16 add a rounding each, so
 // where one part a unit fills the compute units the range stays whole, although
@@ -154,7 +155,7 @@ __device__ __forceinline__ unsigned short gated_bf16(float o, unsigned short g) 
 enum class Second { kRound, kHalfRound, kFree };
 
 inline long long pick_splits(long long units, long long tiles, long long max_splits, bool fp32_parts,
-                             Second second = Second::kRound) {
+                             double merge = 6.0, Second second = Second::kRound) {
   const long long cus = compute_units();
   if (!fp32_parts && units >= cus) return 1;
   if (second == Second::kFree && tiles > 10) return std::max(1LL, std::min((cus + units - 1) / units, max_splits));
@@ -169,7 +170,7 @@ inline long long pick_splits(long long units, long long tiles, long long max_spl
   for (int rounds = 1; rounds <= 3; ++rounds) {
     const long long s = std::min(rounds * cus / units, max_splits);
     if (s <= 1) continue;
-    const double cost = (double)((tiles + s - 1) / s + 12) * rounds_of(units * s) + 6.0;
+    const double cost = (double)((tiles + s - 1) / s + 12) * rounds_of(units * s) + merge;
     if (cost < best_cost) {
       best = s;
       best_cost = cost;

@@ -360,10 +360,11 @@ class MQADecoder:
         chosen = None
         if cfg.chooses(i):  # the top_k rows outside the window by the largest max_h log-softmax weight
             o, lse = kernels.verify_attention(q, keys, values, positions, c ** -0.5, lse=True, from_positions=True,
-                                              out_fm=fm)
+                                              out_fm=fm, captured=True)
             chosen = kernels.choose_rows(q, keys, positions, lse, c ** -0.5, cfg.top_k, cfg.window)
         else:
-            o = kernels.verify_attention(q, keys, values, positions, c ** -0.5, from_positions=True, out_fm=fm)
+            o = kernels.verify_attention(q, keys, values, positions, c ** -0.5, from_positions=True, out_fm=fm,
+                                         captured=True)  # a decoder's steady steps are graphs
         self._attention_out(i, h, x, o, xf)
         return keys, values, chosen
 

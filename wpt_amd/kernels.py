@@ -96,7 +96,7 @@ def _sink(sink, H, device):
 
 def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=None, lse=False, splits=0,
                      generic=False, from_positions=False, key_split=False, static_scratch=False, out_fm=False,
-                     rows32=False):
+                     rows32=False, captured=False):
     """MQA attention of q (B, T, H, c) over k, v (B, N, c): query t of row b
     sees rows max(0, p - window + 1) .. min(p, N - 1), p = positions[b, t]
     (window 0: from row 0), and with tree = (tree_base (B,), ancestors (T,)
@@ -112,7 +112,9 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
     blocks (v_mfma_f32_32x32x16_bf16); static_scratch: the allocation-free entry point
     (wptv_verify_attention_static), whose parts live in the library's own
     device array: no workspace is allocated, and calls overlapping on one
-    device race."""
+    device race; captured: the caller's calls are replayed from a graph, where
+    a second launch costs less than from a program (splits 0 may then cut a
+    short range in parts)."""
     B, T, H, c, N = _check_inputs(q, k, v, positions)
     device = q.device
     library = _lib.lib()
@@ -131,7 +133,7 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
             raise ValueError(f"tree must be (tree_base (B={B},), ancestors (T={T},))")
     flags = ((_lib.FORCE_GENERIC if generic else 0) | (_lib.RANGE_FROM_POSITIONS if from_positions else 0)
              | (_lib.KEY_SPLIT if key_split else 0) | (_lib.OUT_FM if out_fm else 0)
-             | (_lib.ROWS32 if rows32 else 0))
+             | (_lib.ROWS32 if rows32 else 0) | (0 if captured else _lib.CALL_BY_CALL))
     parts, size = _lib.plan("wptv_attention_workspace", "verify_attention", B, T, H, c, N, int(window), dtype, flags,
                             splits=int(splits))
     out = torch.empty_like(q_)
