@@ -8,7 +8,7 @@ from pathlib import Path
 
 import pytest
 
-from wpt_amd import _lib
+from wpt_amd import _lib, layers
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "wptv.h"
 
@@ -96,3 +96,11 @@ def test_the_parts_at_head_width_64(B, T, H, N, parts):
 def test_short_ranges_are_cut_for_graphs_and_left_whole_for_calls_one_by_one(B, T, c, N, parts, alone):
     assert chosen_parts(B, T, 16, c, N) == parts
     assert chosen_parts(B, T, 16, c, N, flags=_lib.RANGE_FROM_POSITIONS | _lib.CALL_BY_CALL) == alone
+
+
+def test_a_reading_whose_stream_passes_4_gb_keeps_the_product_it_had():
+    # wptv_gemm_wide_swiglu refuses operands of 4 GB and more, hipBLASLt does not
+    assert layers.swiglu_tiles(976562, 11264, 2048)
+    assert not layers.swiglu_tiles(976563, 11264, 2048)
+    assert _lib.lib().wptv_gemm_wide_swiglu(16, 2048, 16, 2048, 976563, 11264, 2048, 16, 5632, None) == -3
+    assert b"4 GB" in _lib.lib().wptv_last_error()

@@ -262,9 +262,9 @@ class MQADecoder:
             act = layers.swiglu(F.linear(x, w[f"layers.{i}.gate_up"]))
         elif B * T <= layers.LINEAR_MAX_ROWS:
             act = layers.linear_swiglu(x, w[f"layers.{i}.gate_up_tiles"])  # SwiGLU in the product's epilogue
-        elif layers.wide_tiles(B * T, 2 * self.config.ffn, self.config.d_model):  # a prompt's reading
+        elif layers.swiglu_tiles(B * T, 2 * self.config.ffn, self.config.d_model):  # a prompt's reading
             act = layers.linear_swiglu_wide(x, w[f"layers.{i}.gate_up_tiles"])
-        else:  # widths the tiles do not divide: the product, then SwiGLU of its tile-interleaved halves
+        else:  # no such form: the product, then SwiGLU of its tile-interleaved halves
             gu = F.linear(x, w[f"layers.{i}.gate_up_tiles"]).unflatten(-1, (-1, 2, 32))
             act = (F.silu(gu[..., 0, :].float()) * gu[..., 1, :].float()).flatten(-2).to(x.dtype)
         down = w[f"layers.{i}.down"]

@@ -184,6 +184,13 @@ def wide_tiles(M, N, K):
     return M >= WIDE_MIN_ROWS and N % 256 == 0 and K % 32 == 0
 
 
+def swiglu_tiles(M, N, K):
+    """Whether a gate/up product of M rows (N = 2F) has a form on the 256 x 256
+    tiles with SwiGLU in it (linear_swiglu_wide): operands of 4 GB and more have
+    none."""
+    return wide_tiles(M, N, K) and 2 * K * max(M, N) < 4_000_000_000
+
+
 def linear(x, w, out_dtype=None, splits=0):
     """x (..., K) . w (N, K)^T on the matrix cores (the projections' and the
     lm_head's nn.Linear under bf16 autocast): bf16 operands, FP32
