@@ -104,3 +104,12 @@ def test_a_reading_whose_stream_passes_4_gb_keeps_the_product_it_had():
     assert not layers.swiglu_tiles(976563, 11264, 2048)
     assert _lib.lib().wptv_gemm_wide_swiglu(16, 2048, 16, 2048, 976563, 11264, 2048, 16, 5632, None) == -3
     assert b"4 GB" in _lib.lib().wptv_last_error()
+
+
+@pytest.mark.parametrize("M, N, K, faster", [
+    (513, 11264, 2048, True), (1281, 11264, 2048, True), (4096, 11264, 2048, True), (1281, 22016, 4096, True),
+    (513, 5632, 1024, True), (2000, 768, 256, True), (1000, 2048, 512, True),
+    (1000, 4096, 2048, False), (513, 22016, 4096, False), (513, 2048, 512, False), (1000, 768, 256, False)])
+def test_a_gate_up_product_of_few_tiles_stays_off_them(M, N, K, faster):
+    # measured on the MI355X at these sizes (layers.swiglu_tiles)
+    assert layers.swiglu_tiles(M, N, K) == faster

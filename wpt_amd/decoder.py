@@ -38,9 +38,10 @@ On the GPU:
                     SPLIT_K_ROWS bf16 rows (summed by qkv_post and the
                     residual add + norm), the gate/up product with SwiGLU in
                     its epilogue (wptv_gemm_swiglu at up to 512 bf16 rows,
-                    the 256 x 256 tiles of wptv_gemm_wide_swiglu above);
+                    the 256 x 256 tiles of wptv_gemm_wide_swiglu above
+                    where they are the faster);
                     the lm_head on wptv_gemm (the skinny products up to 320
-                    rows, the 256 x 256 tiles above); hipBLASLt only for a
+                    rows, the 256 x 256 tiles above); hipBLASLt for a
                     prefill's wider layer products
     window layers   wptv_window_qkv_post (norms, rotary encoding, the ring
                     append), wptv_window_attention over the cache's ring with
@@ -264,7 +265,7 @@ class MQADecoder:
             act = layers.linear_swiglu(x, w[f"layers.{i}.gate_up_tiles"])  # SwiGLU in the product's epilogue
         elif layers.swiglu_tiles(B * T, 2 * self.config.ffn, self.config.d_model):  # a prompt's reading
             act = layers.linear_swiglu_wide(x, w[f"layers.{i}.gate_up_tiles"])
-        else:  # no such form: the product, then SwiGLU of its tile-interleaved halves
+        else:  # few tiles, or none: the product, then SwiGLU of its tile-interleaved halves
             gu = F.linear(x, w[f"layers.{i}.gate_up_tiles"]).unflatten(-1, (-1, 2, 32))
             act = (F.silu(gu[..., 0, :].float()) * gu[..., 1, :].float()).flatten(-2).to(x.dtype)
         down = w[f"layers.{i}.down"]

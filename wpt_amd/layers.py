@@ -185,10 +185,20 @@ def wide_tiles(M, N, K):
 
 
 def swiglu_tiles(M, N, K):
-    """Whether a gate/up product of M rows (N = 2F) has a form on the 256 x 256
-    tiles with SwiGLU in it (linear_swiglu_wide): operands of 4 GB and more have
-    none."""
-    return wide_tiles(M, N, K) and 2 * K * max(M, N) < 4_000_000_000
+    """Whether a gate/up product of M rows (N = 2F) is the faster in one
+    launch of 256 x 256 tiles (linear_swiglu_wide) than as torch's product and
+    the SwiGLU of its halves.  A round of tiles, one a compute unit of 256,
+    takes time in proportion to K however few the tiles are, so it pays from
+    some multiple of 65536 results on, and a second round of a few tiles needs
+    more of them.  Measured, us, this and the product: 513 x 11264 x 2048 58, 65;
+    1000 x 4096 x 2048 51, 47; 513 x 2048 x 512 25, 23, 1000 rows 25, 28; 513 x 768
+    x 256 21, 17, 2000 rows 21, 24; two rounds, 513 x 22016 x 4096 186, 160, 768
+    rows 197, 210, 1281 x 11264 x 2048 114, 121.  Operands of 4 GB and more have
+    no such form."""
+    if not wide_tiles(M, N, K) or 2 * K * max(M, N) >= 4_000_000_000:
+        return False
+    rounds = -(-(-(-M // 256) * (N // 256)) // 256)
+    return M * N >= 65536 * (12 + K / 32) * (0.4 + 0.6 * rounds)
 
 
 def linear(x, w, out_dtype=None, splits=0):
