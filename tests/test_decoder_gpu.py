@@ -453,3 +453,12 @@ def test_a_model_folder_loads_the_decoder_it_saved(device, tmp_path):
     loaded = folder.load_decoder(tmp_path, dtype=torch.bfloat16)
     built = MQADecoder(config, weights, dtype=torch.bfloat16)
     assert torch.equal(loaded(ids), built(ids))
+
+
+@pytest.mark.parametrize("T", [5, 161, 200, 288, 330])
+def test_a_decoder_of_head_width_256_reads_any_number_of_rows(device, T):
+    # its attention has no form that writes the fm layout: every row count reads on the row-major products
+    config = DecoderConfig(layers=2, d_model=256, heads=4, head_dim=256, ffn=512, vocab=1024)
+    gpu, ora = models(config, torch.bfloat16)
+    ids = torch.randint(config.vocab, (1, T), generator=torch.Generator().manual_seed(T))
+    assert close(gpu(ids.to(device)).cpu(), ora.forward(ids), 2e-2)

@@ -219,10 +219,11 @@ class MQADecoder:
 
     def fm_rows(self, rows):
         """Whether a reading of `rows` rows runs the fm products (bf16, up to
-        320 rows, every layer's shapes taken by a kernel form)."""
+        320 rows, a head width whose attention writes the fm layout, every
+        layer's shapes taken by a kernel form)."""
         ok = self._fm_rows.get(rows)
         if ok is None:
-            ok = self.dtype == torch.bfloat16 and all(
+            ok = self.dtype == torch.bfloat16 and self.config.head_dim in (64, 128) and all(
                 layers.fm_plan(rows, w.shape[0], w.shape[1], swiglu=name.endswith("gate_up_tiles"),
                                any_rows=True) is not None
                 for name, w in self.fm.items())
