@@ -476,7 +476,7 @@ def projections(model, rows, steps, warmup):
     device = model.device
     generator = torch.Generator(device=device).manual_seed(7)
     out = {}
-    fm = model.fm_rows(rows)  # the step's products at these rows: the fm ones, or the row-major split-K ones
+    fm = model.fm_rows(rows, any_rows=True)  # the step's products at these rows: the fm ones, or the row-major split-K ones
     kinds = [("qkv", cfg.d_model, "split-K (parts)"), ("out", cfg.heads * cfg.head_dim, "split-K (parts)"),
              ("gate_up_tiles", cfg.d_model, "SwiGLU in the epilogue"), ("down", cfg.ffn, "split-K (parts)")]
     for name, K, engine in kinds:
@@ -486,9 +486,9 @@ def projections(model, rows, steps, warmup):
             xf = layers.fm_pack(x)
             ws = [model.fm[f"layers.{i}.{name}"] for i in range(cfg.layers)]
             if name == "gate_up_tiles":
-                calls = [lambda w=w: layers.linear_fm_swiglu(xf, rows, w) for w in ws]
+                calls = [lambda w=w: layers.linear_fm_swiglu(xf, rows, w, any_rows=True) for w in ws]
             else:
-                calls = [lambda w=w: layers.linear_fm_parts(xf, rows, w) for w in ws]
+                calls = [lambda w=w: layers.linear_fm_parts(xf, rows, w, any_rows=True) for w in ws]
         else:
             ws = [model.w[f"layers.{i}.{name}"] for i in range(cfg.layers)]
             if name == "gate_up_tiles":

@@ -106,7 +106,7 @@ def test_fm_swiglu_feeds_the_down_product(device, M):
 
 
 def test_rows_without_a_kernel_form_have_no_plan():
-    # 161 to 288 rows (11 to 18 row blocks) and above 320: the decoder reads them on the row-major products
+    # above 320 rows; 161 to 288 (11 to 18 row blocks) but for the any_rows products, which the decoder reads them on
     assert layers.fm_plan(200, 2048, 2048) is None and layers.fm_plan(288, 2048, 2048) is None
     assert layers.fm_plan(321, 2048, 2048) is None
     assert layers.fm_plan(289, 2048, 2048) is not None and layers.fm_plan(160, 2048, 2048) is not None

@@ -5,10 +5,13 @@ here)."""
 import ctypes
 import re
 from pathlib import Path
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from wpt_amd import _lib, layers
+from wpt_amd.decoder import LARGE, MQADecoder
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "wptv.h"
 
@@ -113,3 +116,16 @@ def test_a_reading_whose_stream_passes_4_gb_keeps_the_product_it_had():
 def test_a_gate_up_product_of_few_tiles_stays_off_them(M, N, K, faster):
     # measured on the MI355X at these sizes (layers.swiglu_tiles)
     assert layers.swiglu_tiles(M, N, K) == faster
+
+
+@pytest.mark.parametrize("rows", [1, 160, 161, 235, 288, 289, 320, 321])
+@pytest.mark.parametrize("any_rows", [False, True])
+def test_the_decoder_s_answer_about_fm_rows_is_the_products(rows, any_rows):
+    # a program that asks fm_rows and then calls the products without any_rows must not be refused
+    shapes = {"qkv": (2304, 2048), "out": (2048, 2048), "gate_up_tiles": (11264, 2048), "down": (2048, 5632)}
+    model = SimpleNamespace(dtype=torch.bfloat16, config=LARGE, _fm_rows={},
+                            fm={f"layers.0.{name}": SimpleNamespace(shape=shape) for name, shape in shapes.items()})
+    taken = all(layers.fm_plan(rows, *shape, swiglu=name == "gate_up_tiles", any_rows=any_rows) is not None
+                for name, shape in shapes.items())
+    assert taken == (rows <= 160 or 289 <= rows <= 320 or any_rows and rows <= 320)
+    assert MQADecoder.fm_rows(model, rows, *([True] if any_rows else [])) == taken

@@ -234,7 +234,8 @@ int fm_plan(int M, int N, int K, bool swiglu, bool halves, int requested, FmPlan
     p->nb = 4;
     p->groups = 2;
   } else if (rb > 10) {
-    return fail(WPTV_E_UNSUPPORTED, "gemm_fm: %d rows have no kernel form (up to 160, or 289 to 320)", M);
+    return fail(WPTV_E_UNSUPPORTED, "gemm_fm: %d rows have no kernel form at N = %d (%s)", M, N,
+                halves ? "161 to 288 rows take multiples of 64, 289 to 320 wider ones" : "up to 160, or 289 to 320");
   }
   p->splits = s;
   p->steps = quarter / s;

@@ -217,17 +217,19 @@ class MQADecoder:
         ring = cache.ring_rows
         return None if ring is None else ring - self.config.window + 1
 
-    def fm_rows(self, rows):
+    def fm_rows(self, rows, any_rows=False):
         """Whether a reading of `rows` rows runs the fm products (bf16, up to
-        320 rows, a head width whose attention writes the fm layout, every
-        layer's shapes taken by a kernel form)."""
-        ok = self._fm_rows.get(rows)
+        160 rows or 289 to 320, a head width whose attention writes the fm
+        layout, every layer's shapes taken by a kernel form); any_rows: as the
+        products called with any_rows, 161 to 288 rows too (the decoder's own
+        readings)."""
+        ok = self._fm_rows.get((rows, any_rows))
         if ok is None:
             ok = self.dtype == torch.bfloat16 and self.config.head_dim in (64, 128) and all(
                 layers.fm_plan(rows, w.shape[0], w.shape[1], swiglu=name.endswith("gate_up_tiles"),
-                               any_rows=True) is not None
+                               any_rows=any_rows) is not None
                 for name, w in self.fm.items())
-            self._fm_rows[rows] = ok
+            self._fm_rows[rows, any_rows] = ok
         return ok
 
     def _attn_input_fm(self, i, fm):
@@ -415,7 +417,7 @@ class MQADecoder:
         x = torch.empty_like(h)
         positions = torch.empty(B, T, dtype=torch.long, device=self.device)
         # the fm products' operand: x in the fragment-major layout
-        xf = layers.fm_empty(B * T, D, self.device) if self.fm_rows(B * T) else None
+        xf = layers.fm_empty(B * T, D, self.device) if self.fm_rows(B * T, any_rows=True) else None
         first_fm = self._attn_input_fm(0, xf is not None)
         # the embedding, the first norm and each token's position in one pass
         layers.embed_rms_norm(ids.contiguous(), self.w["embedding"], self.w["layers.0.attn_norm"], h,
