@@ -157,3 +157,66 @@ def test_a_caller_without_a_workspace_and_the_static_entry(device):
             _lib.dtype_code(qd.dtype), _lib.ptr(pd), 0, None, None, None, B, T, H, c, N, ctypes.c_float(c ** -0.5),
             splits, 0, _lib.ptr(out), None, None, 0, _lib.stream(qd.device)), "verify_attention")
         check(out, expected)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("c", [64, 128])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_values_out_of_sight_in_every_form(device, c, splits, bad):
+    """The visible rows of a tile alone, at both widths' column layouts and in parts: a row that only the last
+    query of batch row 0 sees, and rows nobody sees, hold no number."""
+    B, T, H, N = 2, 5, 4, 200
+    g, q, k, v, _ = inputs(B, T, H, c, N, seed=7)
+    positions = torch.tensor([[150, 151, 152, 153, 154], [10, 11, 12, 13, 14]])
+    expected, _ = formula(q, k, v, causal(positions, N), c ** -0.5)
+    vd = v.clone()
+    vd[0, 154:], vd[1, 15:] = bad, bad
+    got = kernels.verify_attention(q.to(device), k.to(device), vd.to(device), positions.to(device), c ** -0.5,
+                                   splits=splits)
+    assert not torch.isfinite(got[0, 4]).any()
+    got[0, 4] = expected[0, 4].float().to(device)
+    check(got, expected)
+
+
+@pytest.mark.parametrize("splits", [0, 1, 2])
+@pytest.mark.parametrize("c", [64, 128])
+def test_a_tree_branch_never_reads_its_siblings_values(device, c, splits):
+    """Two branches under one root: the left one's value and key rows hold no number; the right one sees none of it."""
+    B, H, prefix = 2, 4, 75
+    parents = [-1, 0, 0, 1, 2, 3, 4]  # root; left 1 3 5; right 2 4 6
+    g, q, k, v, _ = inputs(B, len(parents), H, c, prefix + len(parents), seed=8)
+    seen = torch.zeros(len(parents), prefix + len(parents), dtype=torch.bool)
+    seen[:, :prefix] = True
+    for i, parent in enumerate(parents):
+        if parent >= 0:
+            seen[i, prefix:] = seen[parent, prefix:]
+        seen[i, prefix + i] = True
+    expected, _ = formula(q, k, v, seen.expand(B, -1, -1), c ** -0.5)
+    kd, vd = k.clone(), v.clone()
+    for i in (1, 3, 5):
+        kd[:, prefix + i], vd[:, prefix + i] = float("nan"), float("nan")
+    base = torch.full((B,), prefix, device=device)
+    masks = kernels.tree_ancestors(parents).to(device)
+    got = kernels.verify_attention(q.to(device), kd.to(device), vd.to(device), None, c ** -0.5, tree=(base, masks),
+                                   splits=splits)
+    assert not torch.isfinite(got[:, [1, 3, 5]]).any()
+    got[:, [1, 3, 5]] = expected[:, [1, 3, 5]].float().to(device)
+    check(got, expected)
+
+
+@pytest.mark.parametrize("c", [64, 128])
+def test_a_ring_slot_outside_the_window_may_hold_anything(device, c):
+    """Slots of tokens before the window of every query, and between two queries' windows, hold no number."""
+    B, T, H, window, past = 2, 3, 4, 32, 300
+    g, q, k, v, positions = inputs(B, T, H, c, past + T, seed=9)
+    sink = torch.randn(H, generator=g)
+    expected, _ = formula(q, k, v, causal(positions, past + T, window), c ** -0.5, sink)
+    ring = torch.full((B, 64, 2 * c), float("nan"))
+    held = torch.arange(past - window + 1, past + T)
+    ring[:, held % 64] = torch.cat([k, v], -1)[:, held]
+    ring[:, (past - window + 1) % 64, c:] = float("inf")  # the first query's first row, the others' none
+    got = kernels.ring_attention(q.to(device), ring.to(device), positions.to(device), c ** -0.5, window,
+                                 sink.to(device))
+    assert not torch.isfinite(got[:, 0]).any()
+    got[:, 0] = expected[:, 0].float().to(device)
+    check(got, expected)
