@@ -97,6 +97,10 @@ const char* wptv_last_error(void);
  *              into (0 = chosen from B, T, N and the GPU); the workspace must
  *              hold wptv_attention_workspace() bytes for the same arguments
  *              (FP32 calls with a smaller one, or none, run in one part)
+ *              The count chosen for 0 follows B, T and N, and the order of a
+ *              query's sums follows the count: a query's last bits may differ
+ *              from one batch size or table length to another, in FP32 too.
+ *              With splits 1 they are the same in any batch and table
  *   out        [B, T, H, c] contiguous, dtype
  *   lse        NULL, or [B, T, H] fp32: each query head's natural-log
  *              log-sum-exp, the sink included

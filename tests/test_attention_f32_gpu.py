@@ -220,3 +220,18 @@ def test_a_ring_slot_outside_the_window_may_hold_anything(device, c):
     assert not torch.isfinite(got[:, 0]).any()
     got[:, 0] = expected[:, 0].float().to(device)
     check(got, expected)
+
+
+def test_one_part_gives_a_query_the_same_bits_in_any_batch_and_table(device):
+    """The library's own part count follows the batch and the table's length, and the sums' order with it."""
+    B, T, H, c, N = 6, 5, 4, 64, 500
+    g, q, k, v, positions = inputs(B, T, H, c, N, seed=10)
+    table = torch.cat([k, v], -1).to(device)
+    qd, pd = q.to(device), positions.to(device)
+    whole = kernels.verify_attention(qd, table[..., :c], table[..., c:], pd, c ** -0.5, splits=1)
+    longer = torch.cat([table, torch.zeros(B, 700, 2 * c, device=device)], 1)
+    for b in range(B):
+        for t in (table, longer):
+            one = t[b:b + 1]
+            alone = kernels.verify_attention(qd[b:b + 1], one[..., :c], one[..., c:], pd[b:b + 1], c ** -0.5, splits=1)
+            assert torch.equal(alone[0], whole[b])

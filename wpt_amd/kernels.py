@@ -105,7 +105,9 @@ def verify_attention(q, k, v, positions, scale, *, window=0, sink=None, tree=Non
     tree_base[b] + t); sink (H,) joins each head's softmax denominator.
     Returns the output (B, T, H, c) in q's dtype, and with lse=True also the
     (B, T, H) FP32 log-sum-exp.  splits: key-range parts per batch row (0:
-    the library chooses); generic: the wave-per-query kernel; from_positions:
+    the library chooses, by the batch and the table's length, which the order
+    of a query's sums then follows; with 1 a query's bits are the same in any
+    batch and table); generic: the wave-per-query kernel; from_positions:
     read only the rows the positions reach (a cache table with spare rows);
     key_split: where T*H <= 80, the key-parallel MFMA kernel instead of the
     row-block one; rows32: at head width 128, the row-block kernel on 32-row
