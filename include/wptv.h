@@ -417,7 +417,7 @@ int wptv_gemm_fm_parts(const void* x_fm, const void* w_fm, int M, int N, int K, 
 int wptv_gemm_fm_swiglu(const void* x_fm, const void* w_fm, int M, int N, int K, void* out_fm, hipStream_t stream);
 
 /* wptv_gemm_fm_any_plan, _parts, _swiglu: the same for every row count up to
- * 320 (161 to 288 rows in two row groups). */
+ * 320 (161 to 288 rows in two to four row groups). */
 int wptv_gemm_fm_any_plan(int M, int N, int K, int swiglu, int* splits, size_t* parts_bytes);
 int wptv_gemm_fm_any_parts(const void* x_fm, const void* w_fm, int M, int N, int K, int splits, float* parts,
                            size_t parts_bytes, hipStream_t stream);

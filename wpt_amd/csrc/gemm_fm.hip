@@ -168,11 +168,11 @@ bool fm_steps_built(int s) {
 
 struct FmPlan {
   int mb, nb, splits, steps;
-  int groups;  // row groups of mb row blocks: 1 up to 128 rows, else 2 or 4
+  int groups;  // row groups of mb row blocks: 1 up to 128 rows, else 2 to 4
   size_t bytes;
 };
 
-// halves: 161 to 288 rows are taken too, in two row groups.
+// halves: 161 to 288 rows are taken too, in two to four row groups.
 int fm_plan(int M, int N, int K, bool swiglu, bool halves, int requested, FmPlan* p) {
   if (M <= 0 || N <= 0 || K <= 0)
     return fail(WPTV_E_INVALID, "gemm_fm: M, N and K must be positive (got %d, %d, %d)", M, N, K);
@@ -223,16 +223,17 @@ int fm_plan(int M, int N, int K, bool swiglu, bool halves, int requested, FmPlan
     p->groups = 4;
   } else if (halves && rb > 10 && rb < 20 && N % 64 == 0) {
     // 161 to 288 rows: halves by 64 columns, the most rows that share a
-    // workgroup's weights.  Measured on the MI355X with cold weights, q/k/v, output,
-    // gate/up, down in us, against the row-major products: 235 rows 7.8, 6.4,
-    // 27.5, 13.0 against 11.0, 11.2, 36.4, 15.1 (traced); of the other
-    // tilings (rows of 3, 4, 6 blocks by 32, 64 or 128 columns) none was more
-    // than 0.7 us faster at a product; the gate/up product by row groups of four
-    // blocks, two workgroups a compute unit, takes the same: 192 rows 24.7 against
-    // 24.8, 256 rows 26.6 against 26.7
-    p->mb = rb / 2;
+    // workgroup's weights; the SwiGLU form by groups of four row blocks where four
+    // divide them, the most that leave a compute unit two workgroups (64 KiB of
+    // LDS each).  Measured on the MI355X with cold weights, q/k/v, output, gate/up,
+    // down in us, against the row-major products: 235 rows 7.8, 6.4, 27.5, 13.0
+    // against 11.0, 11.2, 36.4, 15.1 (traced); gate/up in fours and in halves: 161
+    // rows 23.3, 25.2, 192 rows 23.2, 24.8, 225 rows 27.1, 29.1, 256 rows 26.8,
+    // 28.8; of the other tilings (rows of 3, 4, 6 blocks by 32, 64 or 128
+    // columns) none was more than 0.7 us faster at a product
+    p->mb = swiglu && rb % 4 == 0 ? 4 : rb / 2;
     p->nb = 4;
-    p->groups = 2;
+    p->groups = rb / p->mb;
   } else if (rb > 10) {
     return fail(WPTV_E_UNSUPPORTED, "gemm_fm: %d rows have no kernel form at N = %d (%s)", M, N,
                 halves ? "161 to 288 rows take multiples of 64, 289 to 320 wider ones" : "up to 160, or 289 to 320");
@@ -269,6 +270,7 @@ int launch_fm(const FmPlan& p, hipStream_t stream, const void* x, const void* w,
   const dim3 grid(N / (16 * p.nb), p.splits, p.groups);
   if (p.groups > 1 && p.mb != 5) {
     switch (p.mb) {
+      case 4: return launch_fm_steps<4, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
       case 6: return launch_fm_steps<6, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
       case 7: return launch_fm_steps<7, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
       case 8: return launch_fm_steps<8, 4, OUT>(p.steps, grid, stream, x, w, NBT, RBT, M, N, out);
