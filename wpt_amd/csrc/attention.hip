@@ -536,28 +536,33 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_mfma(
   if (splits == 1) {
     typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
     unsigned short* orow = out + ((int64_t)b * R + r) * C;
-    const unsigned short* grow = gate.row<unsigned short>(b, T, r, H, C);
+    const unsigned short* grow = TREE ? nullptr : gate.row<unsigned short>(b, T, r, H, C);  // trees have no gate
     // out_fm > 0: the output [B T, H C] in the fm layout with out_fm row blocks
     const int fm_row = b * T + r / H, fm_col = (r % H) * C;
-    // every gate value before the first store: where it is used, each load waited for the store before it
-    u16x4 gv[G::kCBlocks];
-    if (grow) {
-#pragma unroll
-      for (int cb = 0; cb < G::kCBlocks; ++cb) gv[cb] = *reinterpret_cast<const u16x4*>(grow + cb * 16 + 4 * g);
-    }
-#pragma unroll
-    for (int cb = 0; cb < G::kCBlocks; ++cb) {
-      const f32x4 val = o[cb] * scale_out;
-      u16x4 res;
-      if (grow) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) res[e] = gated_bf16(val[e], gv[cb][e]);
-      } else {
-        res = u16x4{f32_to_bf16(val[0]), f32_to_bf16(val[1]), f32_to_bf16(val[2]), f32_to_bf16(val[3])};
-      }
+    auto store = [&](int cb, u16x4 res) {
       unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + cb * 16 + 4 * g, out_fm)
                                    : orow + cb * 16 + 4 * g;
       *reinterpret_cast<u16x4*>(dst) = res;
+    };
+    if (grow) {
+      // every gate value before the first store: where it is used, each load waited for the store before it.
+      // The two forms apart, so that the registers of the loop above are the ungated form's
+      u16x4 gv[G::kCBlocks];
+#pragma unroll
+      for (int cb = 0; cb < G::kCBlocks; ++cb) gv[cb] = *reinterpret_cast<const u16x4*>(grow + cb * 16 + 4 * g);
+#pragma unroll
+      for (int cb = 0; cb < G::kCBlocks; ++cb) {
+        u16x4 res;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) res[e] = gated_bf16(o[cb][e] * scale_out, gv[cb][e]);
+        store(cb, res);
+      }
+    } else {
+#pragma unroll
+      for (int cb = 0; cb < G::kCBlocks; ++cb) {
+        const f32x4 val = o[cb] * scale_out;
+        store(cb, u16x4{f32_to_bf16(val[0]), f32_to_bf16(val[1]), f32_to_bf16(val[2]), f32_to_bf16(val[3])});
+      }
     }
     if (lse_out && g == 0) lse_out[(int64_t)b * R + r] = lse2 * kLn2;
   } else {
@@ -921,30 +926,33 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
   typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
   if (splits == 1) {
     unsigned short* orow = out + ((int64_t)b * R + r) * C;
-    const unsigned short* grow = gate.row<unsigned short>(b, T, r, H, C);
+    const unsigned short* grow = TREE ? nullptr : gate.row<unsigned short>(b, T, r, H, C);  // trees have no gate
     const int fm_row = b * T + r / H, fm_col = (r % H) * C;
-    // every gate value before the first store, as verify_attention_mfma (31 queries, 21.4 -> 20.0 us)
-    u16x4 gv[4 * kCB];
-    if (grow) {
+    auto store = [&](int i, u16x4 res) {
+      const int c0 = 8 * i + 4 * h;
+      unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + c0, out_fm) : orow + c0;
+      *reinterpret_cast<u16x4*>(dst) = res;
+    };
+    if (grow) {  // as verify_attention_mfma (batch 16, 31 queries: loads where used 14.6, all first 12.7 us)
+      u16x4 gv[4 * kCB];
 #pragma unroll
       for (int i = 0; i < 4 * kCB; ++i) gv[i] = *reinterpret_cast<const u16x4*>(grow + 8 * i + 4 * h);
-    }
 #pragma unroll
-    for (int cb = 0; cb < kCB; ++cb)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int c0 = 32 * cb + 8 * a + 4 * h;
+      for (int i = 0; i < 4 * kCB; ++i) {
         u16x4 res;
-        if (grow) {
 #pragma unroll
-          for (int m = 0; m < 4; ++m) res[m] = gated_bf16(o[cb][4 * a + m] * scale_out, gv[4 * cb + a][m]);
-        } else {
-#pragma unroll
-          for (int m = 0; m < 4; ++m) res[m] = f32_to_bf16(o[cb][4 * a + m] * scale_out);
-        }
-        unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + c0, out_fm) : orow + c0;
-        *reinterpret_cast<u16x4*>(dst) = res;
+        for (int m = 0; m < 4; ++m) res[m] = gated_bf16(o[i / 4][4 * (i % 4) + m] * scale_out, gv[i][m]);
+        store(i, res);
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4 * kCB; ++i) {
+        u16x4 res;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) res[m] = f32_to_bf16(o[i / 4][4 * (i % 4) + m] * scale_out);
+        store(i, res);
+      }
+    }
     if (lse_out && h == 0) lse_out[(int64_t)b * R + r] = lse2 * kLn2;
   } else {
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));

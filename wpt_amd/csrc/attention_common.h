@@ -105,7 +105,7 @@ struct OutGate {
 // lane of the 32-row blocks gates 64 columns): with a division and the rounding
 // in integers a window of 128 took, graph replays, us, in one part and in the two
 // parts that this replaced, then in one part as here: batch 32, 5 queries of 16
-// heads 15.7, 13.3, 11.5; batch 16, 31 queries 21.4, 16.1, 13.2.  The reciprocal is
+// heads 15.7, 13.3, 11.1; batch 16, 31 queries 21.4, 16.1, 12.7.  The reciprocal is
 // v_rcp_f32 of a quarter of the denominator, a quarter of that again, so that a
 // subnormal factor is kept; each of the 65536 gates gives the division's bits.
 __device__ __forceinline__ float round_bf16(float f) { return static_cast<float>(static_cast<__bf16>(f)); }
