@@ -1842,7 +1842,7 @@ int pick_mbw(int R) {
 }
 
 // The window entry points: a gated window in one part is the faster also in a
-// graph (batch 32, 5 queries of 16 heads 11.5 us, 12.6 in two).
+// graph (batch 32, 5 queries of 16 heads 11.1 us, 12.6 in two).
 constexpr int kWindowFlags = WPTV_ATTN_RANGE_FROM_POSITIONS | WPTV_ATTN_CALL_BY_CALL;
 
 // What the combine launch costs the GPU itself, as pick_splits counts it, where
