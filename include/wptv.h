@@ -378,7 +378,7 @@ int wptv_gemm_wide_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw
 
 /* ---------------------------------------------------------------------------
  * The same products with fragment-major ("fm") operands, for the verify
- * step's projections at M <= 160 rows (the reference's nn.Linear under bf16
+ * step's projections at M <= 320 rows (the reference's nn.Linear under bf16
  * autocast: attention.py:157-168, layers.py:45-61).  An fm matrix A [R, K]
  * (bf16, K a multiple of 32) is stored as 1 KiB blocks of 16 rows x 32
  * columns: block (ks, rb) at element (ks * RB + rb) * 512, RB its row-block
@@ -396,7 +396,8 @@ int wptv_gemm_wide_swiglu(const void* x, int64_t ldx, const void* w, int64_t ldw
  * wptv_fm_row_blocks: the row blocks an fm X of M rows has (2 ceil(M / 32)).
  * wptv_gemm_fm_plan: the part count of a product (*splits 0: chosen; in: a
  *   count to check) and the bytes of its FP32 parts; swiglu: the gate/up
- *   form (one part).  N a multiple of 32 (64 for swiglu), K of 128.
+ *   form (one part).  N a multiple of 32 (64 for swiglu), K of 128; M up to
+ *   160, or 289 to 320 (wptv_gemm_fm_any_plan: up to 320).
  * wptv_gemm_fm_parts: parts [splits, M, N] FP32 of x . w^T, each over one
  *   part of K, for a consumer that sums them (wptv_qkv_post_parts,
  *   wptv_add_rms_norm_parts).

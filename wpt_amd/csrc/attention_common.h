@@ -16,9 +16,6 @@ struct Bounds {
   int lo, hi;  // inclusive key-row range a query sees (hi < lo: none)
 };
 
-// The key rows query position t of batch row b sees, before the tree mask.
-// A batch row's query positions: p[t], or (a draft tree given without
-// positions) node t at base + t.
 // p[i] of an input that no kernel of the launch writes, read as constant
 // memory: a scalar load where i is uniform (on the scalar counter, apart from
 // the vector-memory counter the kernels' DMA runs on, which the compiler's own
@@ -28,6 +25,8 @@ __device__ __forceinline__ T const_load(const T* p, int64_t i) {
   return ((const __attribute__((address_space(4))) T*)(uintptr_t)p)[i];
 }
 
+// A batch row's query positions: p[t], or (a draft tree given without
+// positions) node t at base + t.
 struct QueryPos {
   const int64_t* p;
   int64_t base;
@@ -38,6 +37,7 @@ __device__ __forceinline__ QueryPos query_pos(const int64_t* positions, const in
   return positions ? QueryPos{positions + (int64_t)b * T, 0} : QueryPos{nullptr, tree_base[b]};
 }
 
+// The key rows query position t sees, before the tree mask.
 __device__ __forceinline__ Bounds query_bounds(const QueryPos& pos_b, int t, int window, int N) {
   const int64_t p = pos_b.at(t);
   int64_t hi = p < (int64_t)N - 1 ? p : (int64_t)N - 1;

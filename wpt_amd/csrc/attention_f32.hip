@@ -384,7 +384,9 @@ void launch_width(const F32Plan& p, const F32Call& a, float* part_o, float* part
 bool attention_f32_takes(int c) { return c == 64 || c == 128; }
 
 // Whole rounds of one workgroup per compute unit (pick_splits), each wavefront
-// at least one tile.  Measured on the MI355X, graph replays, us a call (batch,
+// at least one tile, so that ranges of nine 32-row tiles and more are cut.  A
+// compute unit holds several workgroups of this kernel; that whole rounds serve
+// is what the table says, not an occupancy.  Measured on the MI355X, graph replays, us a call (batch,
 // queries, heads, width, rows): the wave-per-query kernel, this one with a
 // part more than fills the round, this one
 //   (8, 5, 4, 64, 1029)     366   10.2  10.2

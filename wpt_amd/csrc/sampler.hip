@@ -570,7 +570,10 @@ __global__ __launch_bounds__(kT) void accept_stats(const S* __restrict__ scores,
 // replays of both launches, accept_stats then this, us: k = 5 29.4, 18.4; 40
 // 32.2, 21.4 (in order 38.3, 33.3; FP32 scores 34.1, 21.3); 128 32.6, 26.7; 200
 // 33.2, 30.4 but in order 40.8, 41.3; 1500 40.3, 48.2: with k past a hundred
-// or two some thread of every wavefront has more than two kept entries.
+// or two some thread of every wavefront has more than two kept entries.  Above
+// 32768 entries a thread's 64 spill in both forms (332 bytes of scratch a lane
+// here, 300 there), this one's still the faster: 50257 entries, k = 5 72.4, 47.1; 40
+// 73.0, 61.0; 128 73.2, 68.1 (FP32 82, 46; 82, 56; 82, 66); 65536 alike.
 constexpr int kQuickK = 128;
 
 template <int ITEMS, typename S, bool ORDER>
