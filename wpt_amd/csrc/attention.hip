@@ -928,30 +928,35 @@ __global__ __launch_bounds__(kKeySets * MB * 64, 1) void verify_attention_m32(
     unsigned short* orow = out + ((int64_t)b * R + r) * C;
     const unsigned short* grow = TREE ? nullptr : gate.row<unsigned short>(b, T, r, H, C);  // trees have no gate
     const int fm_row = b * T + r / H, fm_col = (r % H) * C;
-    auto store = [&](int i, u16x4 res) {
-      const int c0 = 8 * i + 4 * h;
-      unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + c0, out_fm) : orow + c0;
-      *reinterpret_cast<u16x4*>(dst) = res;
-    };
     if (grow) {  // as verify_attention_mfma (batch 16, 31 queries: loads where used 14.6, all first 12.7 us)
       u16x4 gv[4 * kCB];
 #pragma unroll
       for (int i = 0; i < 4 * kCB; ++i) gv[i] = *reinterpret_cast<const u16x4*>(grow + 8 * i + 4 * h);
 #pragma unroll
-      for (int i = 0; i < 4 * kCB; ++i) {
-        u16x4 res;
+      for (int cb = 0; cb < kCB; ++cb)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) res[m] = gated_bf16(o[i / 4][4 * (i % 4) + m] * scale_out, gv[i][m]);
-        store(i, res);
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            gv[4 * cb + a][m] = gated_bf16(o[cb][4 * a + m] * scale_out, gv[4 * cb + a][m]);
+#pragma unroll
+      for (int i = 0; i < 4 * kCB; ++i) {
+        const int c0 = 8 * i + 4 * h;
+        unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + c0, out_fm) : orow + c0;
+        *reinterpret_cast<u16x4*>(dst) = gv[i];
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 4 * kCB; ++i) {
-        u16x4 res;
+      for (int cb = 0; cb < kCB; ++cb)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) res[m] = f32_to_bf16(o[i / 4][4 * (i % 4) + m] * scale_out);
-        store(i, res);
-      }
+        for (int a = 0; a < 4; ++a) {
+          const int c0 = 32 * cb + 8 * a + 4 * h;
+          u16x4 res;
+#pragma unroll
+          for (int m = 0; m < 4; ++m) res[m] = f32_to_bf16(o[cb][4 * a + m] * scale_out);
+          unsigned short* dst = out_fm ? out + fm_offset(fm_row, fm_col + c0, out_fm) : orow + c0;
+          *reinterpret_cast<u16x4*>(dst) = res;
+        }
     }
     if (lse_out && h == 0) lse_out[(int64_t)b * R + r] = lse2 * kLn2;
   } else {
