@@ -93,7 +93,8 @@ def test_the_parts_at_head_width_64(B, T, H, N, parts):
 
 @pytest.mark.parametrize("B, T, c, N, parts, alone", [
     (1, 1, 128, 320, 3, 1), (64, 1, 128, 320, 3, 1), (128, 1, 128, 320, 1, 1), (1, 1, 128, 160, 1, 1),  # one block
-    (32, 2, 128, 288, 3, 1), (1, 5, 128, 300, 3, 1), (16, 5, 128, 320, 3, 1), (32, 5, 128, 320, 1, 1),
+    (80, 1, 128, 256, 2, 1), (32, 2, 128, 288, 3, 1), (72, 3, 128, 320, 3, 1), (72, 3, 128, 256, 1, 1),
+    (1, 5, 128, 300, 3, 1), (16, 5, 128, 320, 3, 1), (32, 5, 128, 320, 1, 1),
     (1, 16, 128, 288, 3, 1), (8, 31, 128, 320, 1, 1), (1, 5, 64, 320, 1, 1),
     (1, 5, 128, 700, 6, 6), (32, 5, 128, 4100, 8, 8)])
 def test_short_ranges_are_cut_for_graphs_and_left_whole_for_calls_one_by_one(B, T, c, N, parts, alone):

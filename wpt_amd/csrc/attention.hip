@@ -1852,18 +1852,19 @@ constexpr int kWindowFlags = WPTV_ATTN_RANGE_FROM_POSITIONS | WPTV_ATTN_CALL_BY_
 
 // What the combine launch costs the GPU itself, as pick_splits counts it, where
 // it decides: ranges of 7 to 10 tiles at head width 128, and batches that leave
-// it room beside them.  Measured in graphs, us in one part and in the two (256
-// rows) or three (288 rows and more) that fill the range: up to 16 query rows,
-// batch 1 x 320 10.4, 9.0, 64 x 320 11.2, 10.2, 128 x 320 11.7, 12.2; 17 to 48, 32 x
-// 320 10.7, 9.8; 49 to 128, 1 x 320 11.8, 11.2, 32 x 300 12.8, 13.0; 32-row blocks, 1
-// x 16 x 320 13.9, 12.4, 8 x 31 x 320 14.5, 14.7.  At head width 64 one part is the
-// faster throughout (5 queries of 16 heads, 32 x 320 10.0, 10.8).
+// room for three parts beside each other.  Measured in graphs, us in one part and
+// in the two (up to 256 rows) or three (288 rows and more) that fill the range: up to
+// 16 query rows, batch 1 x 320 10.4, 9.0, 80 x 320 11.6, 10.7, 80 x 256 10.3, 10.1, 127
+// x 320 11.6, 12.4; 17 to 48, 32 x 320 10.7, 9.8, 72 x 288 11.0, 10.7, 72 x 256 10.0,
+// 10.3; 49 to 128, 1 x 320 11.8, 11.2, 32 x 300 12.8, 13.0; 32-row blocks, 1 x 16 x 320
+// 13.9, 12.4, 8 x 31 x 320 14.5, 14.7.  At head width 64 one part is the faster
+// throughout (5 queries of 16 heads, 32 x 320 10.0, 10.8).
 double graph_merge(int c, int R, long long units) {
-  if (c != 128 || units > 64) return 6.0;
+  if (c != 128 || units > compute_units() / 3) return 6.0;
+  const bool few = units <= 16;
   if (R <= 16) return 2.0;
-  if (R <= 48) return 3.0;
-  if (units > 16) return 6.0;
-  return R <= 128 ? 5.0 : 3.0;
+  if (R <= 48) return few ? 3.0 : 4.0;
+  return !few ? 6.0 : R <= 128 ? 5.0 : 3.0;
 }
 
 // max_bytes: the parts of a count of the library's choosing fit in that many.
